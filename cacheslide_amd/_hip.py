@@ -207,6 +207,7 @@ SIGNATURES = {
     "cs_check_positions": (_I32, [_P, _I64, _I32, _P, _P]),
     "cs_check_bias_positions": (_I32, [_VP, _I64, _P, _P]),
     "cs_ccpe_attention": (_I32, [ctypes.POINTER(CsCcpeArgs), _P]),
+    "cs_ccpe_attention_dense": (_I32, [ctypes.POINTER(CsCcpeArgs), _P]),
     "cs_ccpe_prefill_policy_workspace_bytes": (_I64, [_I32, _I32, _I64]),
     "cs_ccpe_prefill_policy_bf16": (_I32, [ctypes.POINTER(CsCcpeArgs), _P, _I64, _P]),
     "cs_prepare_device": (_I32, []),

@@ -584,6 +584,20 @@ def cope_attention(
         ck.finish()
         return output
 
+    if default_keys and _dense_ok(query, key, value, e, cope, amask, visibility_mask, fixed_positions, canonical,
+                                  selected, return_positions):
+        output = torch.empty((nq, hq, value.shape[2]), dtype=value.dtype, device=device)
+        args = _ccpe_args(query, key, value, e, query_positions, None, ck)
+        args.out = _hip.view(output)
+        call("cs_ccpe_attention_dense", args, ck.stream)
+        flags_value = _hip.read_flags(ck.flags)[0]
+        if not flags_value & _hip.FLAG_POLICY_GENERIC:
+            ck.finish(value=flags_value)
+            return output
+        # values near or past the end of the finite range: the generic kernel
+        # decides between the result and the reference's error
+        ck.flags.bitwise_and_(~_hip.FLAG_POLICY_GENERIC)
+
     if fixed_positions is not None:
         call("cs_check_bias_positions", vref(fixed_positions), cope.max_positions, ck.flags_ptr, ck.stream)
 
@@ -739,6 +753,35 @@ def _fast_path_ok(query, key, value, e, cope, amask, visibility_mask, fixed_posi
         return False
     for t in (query, key, value):
         if t.stride(2) != 1 or t.data_ptr() % 16 or t.stride(0) % 8 or t.stride(1) % 8:
+            return False
+    group = query.shape[1] // key.shape[1]
+    return group in (1, 2, 4, 8, 16, 32)
+
+
+def _dense_ok(query, key, value, e, cope, amask, visibility_mask, fixed_positions, canonical, selected,
+              return_positions) -> bool:
+    """The calls of cs_ccpe_attention_dense: f16 and f32 at head size 64 and
+    128, bf16 at 64 (bf16 at 128 has its own kernel, ``_fast_path_ok``)."""
+    d = query.shape[2]
+    if d != 64 and (d != 128 or query.dtype == torch.bfloat16):
+        return False
+    if query.dtype not in (torch.float16, torch.float32, torch.bfloat16):
+        return False
+    if value.shape[2] != d or value.dtype != query.dtype or cope.head_dim != d:
+        return False
+    if amask is not None or visibility_mask is not None or fixed_positions is not None:
+        return False
+    if canonical is not None or selected is not None or return_positions:
+        return False
+    if e.dtype != torch.float32 or not e.is_contiguous() or cope.max_positions > 128:
+        return False
+    if key.shape[0] == 0 or key.shape[0] >= 1 << 30 or query.shape[0] >= 1 << 30:
+        return False
+    per = 16 // query.element_size()
+    for t in (query, key, value):
+        if t.stride(2) != 1 or t.data_ptr() % 16 or t.stride(0) % per or t.stride(1) % per:
+            return False
+        if t.stride(0) < 0 or t.stride(1) < 0:
             return False
     group = query.shape[1] // key.shape[1]
     return group in (1, 2, 4, 8, 16, 32)

@@ -85,7 +85,8 @@ enum cs_flag {
   CS_FLAG_ROW_LOST = 1 << 20,         /* an active token in neither the previous rows nor the snapshot */
   CS_FLAG_ROWS_UNSORTED = 1 << 21,    /* a token list is not ascending and distinct */
   CS_FLAG_ROW_INDEX = 1 << 22,        /* a gather index outside the source rows */
-  /* cs_ccpe_prefill_policy_bf16: the call needs cs_ccpe_attention instead
+  /* cs_ccpe_prefill_policy_bf16, cs_ccpe_attention_dense: the call needs
+   * cs_ccpe_attention instead
      (more dynamic keys beside fixed keys than the path checker holds); its
      results are to be discarded */
   CS_FLAG_POLICY_GENERIC = 1 << 23
@@ -156,6 +157,15 @@ typedef struct cs_ccpe_args {
 } cs_ccpe_args;
 
 int cs_ccpe_attention(const cs_ccpe_args* args, void* stream);
+
+/* The same without masks, fixed positions, policies or traces, on MFMA: dense
+ * q, k, v in f16 or f32 (head size 64 or 128) or bf16 (64), default key
+ * coordinates (kpos null), fp32 table of at most 128 positions, a GQA group
+ * that divides 32, 16-byte aligned rows; CS_EUNSUPPORTED (nothing launched)
+ * otherwise.  Sets CS_FLAG_POLICY_GENERIC in *flags, with out undefined, when
+ * a score, a table product or an output is not finite or beyond 1e37: the
+ * caller runs cs_ccpe_attention instead. */
+int cs_ccpe_attention_dense(const cs_ccpe_args* args, void* stream);
 
 /* cope_attention with the two runtime policies on bf16 MFMA: the reuse call of
  * runtime.py:576-609 (CanonicalPositionPolicy, attention.py:18-57, and/or
