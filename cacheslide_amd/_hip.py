@@ -224,6 +224,7 @@ SIGNATURES = {
          ctypes.POINTER(CsKvSource), _P, _I32, _P, _P, _P],
     ),
     "cs_ccpe_decode_workspace_bytes": (_I64, [_I32, _I32, _I32, _I32]),
+    "cs_ccpe_decode_workspace_best_bytes": (_I64, [_I32, _I32, _I32, _I32]),
     "cs_ccpe_decode_bf16": (
         _I32,
         [_P, _I64, _I64, _I32, _I32, _I32, _P, _I32, ctypes.POINTER(CsKvSource), _P,

@@ -205,7 +205,7 @@ def decode_workspace_bytes(batch: int, heads: int, max_context: int, split: int)
 
 
 def decode_workspace(batch: int, heads: int, max_context: int, split: int, device) -> Tensor:
-    nbytes = decode_workspace_bytes(batch, heads, max_context, split)
+    nbytes = int(_hip.load().cs_ccpe_decode_workspace_best_bytes(batch, heads, max_context, split))
     return torch.empty(max(nbytes, 16), dtype=torch.uint8, device=device)
 
 
@@ -234,8 +234,10 @@ def ccpe_decode_paged(
     ``max_context`` bounds context_lens (read back from the device when
     omitted); a larger context raises ValueError, as does an empty one
     (position.py:149-150).  ``split`` is the number of keys per split-K work
-    item (multiple of 64, <= 1024).  ``workspace`` (uint8, device) must hold
-    ``decode_workspace_bytes(B, Hq, max_context, split)`` bytes.  ``out``
+    item (multiple of 64, <= 1024; fewer keys where a small batch would leave
+    compute units idle and the workspace has room).  ``workspace`` (uint8,
+    device) must hold ``decode_workspace_bytes(B, Hq, max_context, split)``
+    bytes; ``decode_workspace`` gives room for the finer splits too.  ``out``
     (bf16 [B, Hq, 128], contiguous) receives the rows when given.  ``flags``
     (from ``_hip.new_flags``) collects the error bits of this and earlier
     calls when given, for a caller that checks once (``raise_flags``) after a
@@ -381,8 +383,11 @@ class SharedRuns:
 
 def decode_shared_workspace(batch: int, heads: int, shared: SharedRuns, max_context: int, split: int,
                             device) -> Tensor:
-    nbytes = int(_hip.load().cs_ccpe_decode_shared_workspace_bytes(batch, heads, shared.head_items, max_context,
-                                                                      split))
+    lib = _hip.load()
+    nbytes = int(lib.cs_ccpe_decode_shared_workspace_bytes(batch, heads, shared.head_items, max_context, split))
+    # the exact fallback's finer splits (decode_workspace)
+    nbytes += int(lib.cs_ccpe_decode_workspace_best_bytes(batch, heads, max_context, split)
+                  - lib.cs_ccpe_decode_workspace_bytes(batch, heads, max_context, split))
     return torch.empty(max(nbytes, 256) + 256, dtype=torch.uint8, device=device)
 
 

@@ -3,8 +3,8 @@
 // runtime.py:489-508), bf16, head dim 128, K/V from the paged cache.
 //
 // Split-K with speculative saturation.  The keys of a request are cut into
-// splits aligned to the last key (split r covers [nk-(r+1)S, nk-rS)), so the
-// right-most split always holds S keys.  Split 0 is computed exactly (carry 0).
+// splits aligned to the last key: split 0 the last S0 keys, split r > 0 the S
+// keys before split r-1 (plan_splits).  Split 0 is computed exactly (carry 0).
 // Every other split assumes that the gate mass of the keys to its right is
 // already >= P-1, which makes every position in it P-1 and the bias the row
 // constant QE[P-1]; it records its own gate total.  A second launch, one
@@ -83,7 +83,7 @@ struct decode_params {
   kv_addr kv;
   const float* e;
   int32_t npos;
-  int32_t split, smax;
+  int32_t split0, split, smax;  // keys of split 0 and of the others, splits at most
   double* tot;         // [B, hq, smax] gate totals
   double* carry;       // [B, hq, smax] gate mass to the right of each split
   float* mx;           // [B, hq, smax] running max (log2 domain)
@@ -95,6 +95,18 @@ struct decode_params {
   // workgroup): the exact fallback of a shared-chunk decode
   const int32_t* gate;
 };
+
+// Compute units of the current device (cached per device; 256 without one).
+int compute_units() {
+  static int cus[64] = {};
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
+  if (cus[dev] == 0) {
+    int v = 0;
+    cus[dev] = hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && v > 0 ? v : 256;
+  }
+  return cus[dev];
+}
 
 __device__ inline int64_t ws_index(const decode_params& p, int b, int h, int r) {
   return (static_cast<int64_t>(b) * p.hq + h) * p.smax + r;
@@ -137,17 +149,28 @@ __device__ inline int keys_of(const decode_params& p, int b) {
   return nk < p.max_nk ? nk : p.max_nk;
 }
 
+// Splits of nk keys: the right-most split0, then split keys each.
+__device__ inline int splits_of(const decode_params& p, int nk) {
+  if (nk <= 0) return 0;
+  const int splits = nk <= p.split0 ? 1 : 1 + (nk - p.split0 + p.split - 1) / p.split;
+  return splits < p.smax ? splits : p.smax;  // the workspace holds smax splits
+}
+
+// Keys of a wavefront of a split: an equal share, in whole tiles.
+__device__ inline int wave_keys(const split_ctx& c) {
+  return (static_cast<int>(c.hi - c.lo) + kWaves * kTile - 1) / (kWaves * kTile) * kTile;
+}
+
 __device__ inline bool make_ctx(const decode_params& p, int b, int kvh, int r, split_ctx& c) {
   const int nk = keys_of(p, b);
-  int splits = (nk + p.split - 1) / p.split;
-  if (splits > p.smax) splits = p.smax;  // the workspace holds smax splits
-  if (r >= splits) return false;
+  if (r >= splits_of(p, nk)) return false;
   c.b = b;
   c.kvh = kvh;
   c.h0 = kvh * p.group;
   c.r = r;
-  c.hi = static_cast<int64_t>(nk) - static_cast<int64_t>(r) * p.split;
-  c.lo = c.hi - p.split > 0 ? c.hi - p.split : 0;
+  c.hi = r == 0 ? nk : static_cast<int64_t>(nk) - p.split0 - static_cast<int64_t>(r - 1) * p.split;
+  const int64_t keys = r == 0 ? p.split0 : p.split;
+  c.lo = c.hi - keys > 0 ? c.hi - keys : 0;
   return true;
 }
 
@@ -497,7 +520,7 @@ __device__ void run_spec(const decode_params& p, smem_t<G>& s, const split_ctx& 
   const float c_scale = kInvSqrtD * kLog2e;
   __syncthreads();
 
-  const int kw = p.split / kWaves;
+  const int kw = wave_keys(c);
   int64_t wlo = c.lo + static_cast<int64_t>(wave) * kw;
   int64_t whi = wlo + kw;
   if (wlo > c.hi) wlo = c.hi;
@@ -576,14 +599,22 @@ __device__ void run_exact(const decode_params& p, smem_t<G>& s, const split_ctx&
     s.q[h][d] = bf16_to_float(p.q[c.b * p.q_sb + (c.h0 + h) * p.q_sh + d]);
   }
   __syncthreads();
+  // 32 loads in flight: with the compiler's own 4 this sum took 7400 of the
+  // split's 35700 cycles
   for (int i = tid; i < G * p.npos; i += kThreads) {
     const int h = i / p.npos, pp = i % p.npos;
     float a = 0.f;
-    for (int d = 0; d < kD; ++d) a += s.q[h][d] * p.e[d * p.npos + pp];
+    for (int d0 = 0; d0 < kD; d0 += 32) {
+      float ev[32];
+#pragma unroll
+      for (int d = 0; d < 32; ++d) ev[d] = p.e[(d0 + d) * p.npos + pp];
+#pragma unroll
+      for (int d = 0; d < 32; ++d) a += s.q[h][d0 + d] * ev[d];
+    }
     s.qe[h][pp] = a;
   }
 
-  const int kw = p.split / kWaves;
+  const int kw = wave_keys(c);
   int64_t wlo = c.lo + static_cast<int64_t>(wave) * kw;
   int64_t whi = wlo + kw;
   if (wlo > c.hi) wlo = c.hi;
@@ -927,9 +958,7 @@ __global__ void __launch_bounds__(kThreads) decode_finish_kernel(decode_params p
   if (p.gate != nullptr && __builtin_amdgcn_readfirstlane(*p.gate) == 0) return;  // before any barrier
   const int b = blockIdx.x / p.hkv, kvh = blockIdx.x % p.hkv;
   const int h0 = kvh * G;
-  int splits = (keys_of(p, b) + p.split - 1) / p.split;
-  if (splits > p.smax) splits = p.smax;
-  if (splits < 0) splits = 0;  // no key: zero rows (the call is flagged)
+  const int splits = splits_of(p, keys_of(p, b));  // no key: zero rows (the call is flagged)
   bool bad = false;
   if (merge_fast_any<G>(p, s, b, h0, splits)) return;
   fixup_group<G, PAGED>(p, s, b, kvh, bad);
@@ -959,13 +988,57 @@ void launch_group(const decode_params& p, hipStream_t s) {
 
 using namespace cs;
 
+namespace {
+
+// Workspace of one (request, head, split): tot, carry (f64) | acc (f32 x 128) | mx, sm (f32)
+constexpr int64_t kSplitBytes = 8 + 8 + 4 * kD + 4 + 4;
+
+struct split_plan {
+  int32_t split0, split;
+  int64_t smax;
+};
+
+// The splits of a call: `split` keys each while that gives the chip enough
+// workgroups, else `split` halved until it does (128 keys at the least, 32
+// splits at the most: those are merged in one round of loads).  A workgroup
+// draws about 10 bytes a cycle whatever its shape, so a call of few
+// workgroups takes the time of its longest split.  Split 0 keeps at least 4 P
+// keys (and 256): with gates around 1/2 its mass is then twice the P-1 that
+// lets the other splits stand, where a shorter one would leave the next
+// splits to the finish launch, one after another.  The finer plan must fit
+// the workspace (bytes < 0: no limit).
+split_plan plan_splits(int64_t batch, int64_t hq, int64_t hkv, int64_t max_nk, int32_t split, int32_t npos,
+                       int64_t bytes) {
+  split_plan best{split, split, ceil_div(max_nk, split)};
+  const int64_t enough = 2 * static_cast<int64_t>(compute_units());
+  for (int32_t s = split; s >= 256 && s % 128 == 0 && batch * hkv * best.smax < enough;) {
+    s /= 2;
+    int32_t s0 = (4 * npos + 63) / 64 * 64;
+    s0 = s0 < 256 ? 256 : s0;
+    s0 = s0 < s ? s : (s0 > split ? split : s0);
+    const int64_t smax = max_nk <= s0 ? 1 : 1 + ceil_div(max_nk - s0, s);
+    if (smax > 32 || (bytes >= 0 && batch * hq * smax * kSplitBytes > bytes)) break;
+    best = split_plan{s0, s, smax};
+  }
+  return best;
+}
+
+}  // namespace
+
 extern "C" int64_t cs_ccpe_decode_workspace_bytes(int32_t batch, int32_t hq, int32_t max_nk,
                                                   int32_t split) {
   if (batch <= 0 || hq <= 0 || max_nk <= 0 || split <= 0) return 0;
-  const int64_t smax = (static_cast<int64_t>(max_nk) + split - 1) / split;
-  const int64_t n = static_cast<int64_t>(batch) * hq * smax;
-  // tot, carry (f64) | acc (f32 x 128) | mx, sm (f32)
-  return n * (8 + 8 + 4 * kD + 4 + 4);
+  return static_cast<int64_t>(batch) * hq * ceil_div(max_nk, split) * kSplitBytes;
+}
+
+extern "C" int64_t cs_ccpe_decode_workspace_best_bytes(int32_t batch, int32_t hq, int32_t max_nk,
+                                                       int32_t split) {
+  if (batch <= 0 || hq <= 0 || max_nk <= 0 || split <= 0) return 0;
+  // the finest plan of any call of this size: fewest KV heads, smallest split 0
+  const split_plan f = plan_splits(batch, hq, hq < kMaxGroup ? 1 : hq / kMaxGroup, max_nk, split, 2, -1);
+  const int64_t fine = static_cast<int64_t>(batch) * hq * f.smax * kSplitBytes;
+  const int64_t base = cs_ccpe_decode_workspace_bytes(batch, hq, max_nk, split);
+  return fine > base ? fine : base;
 }
 
 namespace {
@@ -1055,7 +1128,7 @@ int prepare_decode(const void* q, int64_t q_s_batch, int64_t q_s_head, int32_t b
   }
   p.e = e;
   p.npos = max_positions;
-  p.split = split;
+  p.split0 = p.split = split;
   p.smax = static_cast<int32_t>(smax);
   p.out = static_cast<uint16_t*>(out);
   p.flags = flags;
@@ -1063,8 +1136,13 @@ int prepare_decode(const void* q, int64_t q_s_batch, int64_t q_s_head, int32_t b
   return CS_OK;
 }
 
-// Carve the workspace of a prepared call and launch its kernels.
-int launch_decode(decode_params& p, void* workspace, void* stream) {
+// Plan the splits of a prepared call over a workspace of `bytes` (at least
+// cs_ccpe_decode_workspace_bytes), carve it and launch the kernels.
+int launch_decode(decode_params& p, void* workspace, int64_t bytes, void* stream) {
+  const split_plan f = plan_splits(p.batch, p.hq, p.hkv, p.max_nk, p.split, p.npos, bytes);
+  p.split0 = f.split0;
+  p.split = f.split;
+  p.smax = static_cast<int32_t>(f.smax);
   const int64_t n = static_cast<int64_t>(p.batch) * p.hq * p.smax;
   char* ws = static_cast<char*>(workspace);
   p.tot = reinterpret_cast<double*>(ws);
@@ -1154,7 +1232,7 @@ extern "C" int cs_ccpe_decode_bf16_noalloc(const void* q, int64_t q_s_batch, int
   if (sst) return sst;
   // every workspace field the kernels read is written earlier in the same call,
   // so the previous call's contents need no clearing
-  return launch_decode(p, ws, stream);
+  return launch_decode(p, ws, CS_DECODE_SCRATCH_BYTES, stream);
 }
 
 extern "C" int cs_ccpe_decode_bf16(const void* q, int64_t q_s_batch, int64_t q_s_head,
@@ -1172,7 +1250,7 @@ extern "C" int cs_ccpe_decode_bf16(const void* q, int64_t q_s_batch, int64_t q_s
   CS_REQUIRE(workspace_bytes >= need, "decode workspace holds %lld bytes, the call needs %lld",
              static_cast<long long>(workspace_bytes), static_cast<long long>(need));
   CS_REQUIRE((reinterpret_cast<uintptr_t>(workspace) % 16) == 0, "workspace must be aligned");
-  return launch_decode(p, workspace, stream);
+  return launch_decode(p, workspace, workspace_bytes, stream);
 }
 
 // ---- decode over shared runs of blocks ---------------------------------------
@@ -1338,5 +1416,5 @@ extern "C" int cs_ccpe_decode_shared_bf16(const cs_decode_shared_args* a, void* 
   // the exact decode over the full block table, run only when some tail left a
   // head's positions below P-1
   p.gate = w.gate;
-  return launch_decode(p, w.decode, stream);
+  return launch_decode(p, w.decode, w.decode_bytes + (workspace_bytes - w.bytes), stream);
 }

@@ -1,0 +1,63 @@
+"""Small decode calls cut finer than ``split`` (fewer workgroups than the chip
+holds): against the oracle at the edges of the splits, with gates around 1/2
+(every later split stands) and near 0 (every split is recomputed), and with a
+workspace that only has room for the caller's own split."""
+
+from __future__ import annotations
+
+import numpy as np
+import pytest
+import torch
+
+from cacheslide_amd import _hip
+from cacheslide_amd.ccpe import ccpe_decode_paged, decode_workspace, decode_workspace_bytes
+from oracle import ccpe as orc
+from tests._helpers import acc_np, assert_close_bf16, fill_paged, paged_layout, seeded
+from tests.test_gpu_ccpe import cope_on
+
+pytestmark = pytest.mark.gpu
+
+
+def setup(device, lens, hq, hkv, npos, low_gates=False):
+    blocks, table, rows = paged_layout(lens, hkv, 16, 128, seed=sum(lens))
+    cache = torch.zeros((blocks, hkv, 16, 256), dtype=torch.bfloat16)
+    keys = [seeded((n, hkv, 128), 7 + i, dtype=torch.bfloat16) for i, n in enumerate(lens)]
+    vals = [seeded((n, hkv, 128), 17 + i, dtype=torch.bfloat16) for i, n in enumerate(lens)]
+    q = seeded((len(lens), hq, 128), 3, dtype=torch.bfloat16)
+    if low_gates:                       # q.k / sqrt(128) around -5: gates of 0.007
+        q = q.abs()
+        keys = [-(k.abs() * 0.7) for k in keys]
+    fill_paged(cache, rows, keys, vals)
+    e = seeded((128, npos), 5, scale=0.1)
+    want = np.concatenate([orc.cope_attention(acc_np(q[i:i + 1]), acc_np(k), acc_np(v), e.numpy(),
+                                              np.array([n - 1]))
+                           for i, (n, k, v) in enumerate(zip(lens, keys, vals))])
+    args = (q.to(device), cache.to(device), table.to(device), torch.tensor(lens, dtype=torch.int32, device=device),
+            cope_on(device, 128, npos, table=e))
+    return args, want
+
+
+@pytest.mark.parametrize("npos", [64, 128])
+@pytest.mark.parametrize("lens", [[1], [255], [256, 257], [384, 385, 511, 513], [1500], [4200, 37]])
+def test_small_calls_match_the_oracle(device, lens, npos):
+    args, want = setup(device, lens, 8, 2, npos)
+    assert_close_bf16(ccpe_decode_paged(*args, max_context=max(lens)), want)
+
+
+@pytest.mark.parametrize("lens", [[700], [1500, 129]])
+def test_small_calls_with_low_gates(device, lens):
+    args, want = setup(device, lens, 8, 1, 64, low_gates=True)
+    assert_close_bf16(ccpe_decode_paged(*args, max_context=max(lens)), want)
+
+
+def test_a_workspace_for_the_plain_split_is_taken(device):
+    lens = [1500]
+    args, want = setup(device, lens, 8, 2, 64)
+    small = torch.empty(decode_workspace_bytes(1, 8, 1500, 1024), dtype=torch.uint8, device=device)
+    assert decode_workspace(1, 8, 1500, 1024, device).numel() > small.numel()
+    guard = torch.full((4096,), 77, dtype=torch.uint8, device=device)
+    both = torch.cat([small, guard])
+    flags = _hip.new_flags(device)
+    out = ccpe_decode_paged(*args, max_context=1500, workspace=both[:small.numel()], flags=flags)
+    assert_close_bf16(out, want)
+    assert bool((both[small.numel():] == 77).all())
