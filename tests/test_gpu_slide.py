@@ -114,6 +114,33 @@ def test_free_list_large_random(device):
     np.testing.assert_array_equal(got.cpu().numpy(), want)
 
 
+@pytest.mark.parametrize("nbits,count", [(1, 1), (33, 20), (2048, 2048), (32_800, 32_769), (70_001, 1), (70_001, 0)])
+def test_free_list_bits_left_after_acquire(device, nbits, count):
+    rng = np.random.default_rng(nbits)
+    free = rng.random(nbits) < 0.6
+    free[rng.permutation(nbits)[:count]] = True
+    fl = relocate.SlotFreeList(nbits, device, free_from=nbits)
+    fl.release(torch.from_numpy(np.flatnonzero(free)).to(device))
+    left = free.copy()
+    want = orc.acquire_lowest(left, count)
+    np.testing.assert_array_equal(fl.acquire(count).cpu().numpy(), want)
+    left[np.asarray(want, dtype=np.int64)] = False
+    np.testing.assert_array_equal(fl.free_mask().numpy(), left)
+
+
+@pytest.mark.parametrize("shape", [(2, 9, 3, 4, 8), (3, 9, 8, 16, 256), (7, 2, 16, 96)])
+def test_page_copy_of_compact_pages(device, shape):
+    """Pages that are one run of bytes, of less than, exactly and more than the
+    bytes a workgroup copies, and ones past the cache's blocks (skipped)."""
+    cache = torch.randn(shape, generator=torch.Generator().manual_seed(5)).to(torch.bfloat16).to(device)
+    blocks = shape[-4]
+    src, dst = torch.tensor([0, 3, 5, blocks]), torch.tensor([6, 1, -1, 2])
+    want = cache.clone()
+    want[..., dst[:2].to(device), :, :, :] = cache[..., src[:2].to(device), :, :, :]
+    relocate.copy_pages(cache, src.to(device), dst.to(device))
+    assert torch.equal(cache, want)
+
+
 # ------------------------------------------------------------ reference fixtures
 def fixture_arena(device, max_selected=2):
     # tests/test_paged.py:13-23 (non-contiguous cache: every second element)
