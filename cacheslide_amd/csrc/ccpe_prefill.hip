@@ -1606,12 +1606,16 @@ extern "C" int cs_ccpe_prefill_policy_bf16(const cs_ccpe_args* a, void* workspac
   src.k_s_head = kv.stride[1];
   src.v_s_tok = vv.stride[0];
   src.v_s_head = vv.stride[1];
+  // With selected rows and a profile (an unsplit walk), the call takes the time
+  // of its few row blocks that see every key: 4 wavefronts a workgroup leave
+  // each a SIMD of its own (512 tiles: 561 us; 8 wavefronts 620, 2 646).
+  const int max_waves = canon && a->sel_rows ? 4 : 8;
   cs::prefill_params p{};
   int waves = 4;
   size_t smem = 0;
   const int st = prepare_prefill(qv.data, 0, qv.stride[0], qv.stride[1], a->qpos, 0, 1, nq, hq, hkv, w.nk_dev,
                                  &src, static_cast<const float*>(ev.data), static_cast<int32_t>(ev.shape[1]),
-                                 a->out.data, a->flags, &p, &waves, &smem);
+                                 a->out.data, a->flags, &p, &waves, &smem, max_waves);
   if (st) return st;
   if (nq == 0) return CS_OK;
   hipStream_t s = as_stream(stream);
@@ -1656,19 +1660,21 @@ extern "C" int cs_ccpe_prefill_policy_bf16(const cs_ccpe_args* a, void* workspac
     p.part_ml = w.part_ml;
     hipLaunchKernelGGL(policy_split_plan_kernel, dim3(1), dim3(kPlanThreads), 0, s, p, w.plan, w.items, w.blocks);
   }
-  // The attention kernel is queued first, so that its longest workgroups
-  // (rows whose walks cover every causal key) are dispatched at once; the
-  // checker, forked after the lowering kernels and the checker's block
-  // descriptors (queued here, ahead of the attention, so that they do not
-  // wait behind it for compute units), then fills the compute units the
-  // attention's short workgroups leave.
-  std::unique_lock<std::mutex> side_lock(g_side_mutex, std::defer_lock);
-  side_lane* side = nullptr;
   if (canon) {
     const int64_t nb = (static_cast<int64_t>(nk) + 255) / 256;
     if (nb > 0)
       hipLaunchKernelGGL(policy_blocks_kernel, dim3(static_cast<uint32_t>((nb + 3) / 4)), dim3(256), 0, s,
                          w.code, static_cast<int64_t>(nk), w.blk);
+  }
+  // The attention kernel is queued first, so that its longest workgroups
+  // (rows whose walks cover every causal key) are dispatched at once; the
+  // checker, forked after the lowering kernels and the checker's block
+  // descriptors (queued above, ahead of the attention, so that they do not
+  // wait behind it for compute units), then fills the compute units the
+  // attention's short workgroups leave.
+  std::unique_lock<std::mutex> side_lock(g_side_mutex, std::defer_lock);
+  side_lane* side = nullptr;
+  if (canon) {
     side_lock.lock();
     const int sst = side_lane_of_current(&side);
     if (sst) return sst;
