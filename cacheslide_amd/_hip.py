@@ -135,6 +135,14 @@ class CsCcpeArgs(ctypes.Structure):
     ]
 
 
+class CsPolicyLowerArgs(ctypes.Structure):
+    """cs_policy_lower_args: both policies' kernel data in one launch."""
+
+    _fields_ = [(name, ctypes.c_int64 if name in ("nq", "nk", "table_size", "n_fixed", "n_selected") else ctypes.c_void_p)
+                for name in ("qpos", "nq", "kpos", "nk", "q_table", "k_table", "table_size", "q_rows", "k_ord",
+                             "fixed", "n_fixed", "selected", "n_selected", "sel_rows", "fixed_keys")]
+
+
 class CsKvSource(ctypes.Structure):
     _fields_ = [
         ("cache", ctypes.c_void_p),
@@ -205,6 +213,8 @@ SIGNATURES = {
     "cs_last_error": (ctypes.c_char_p, []),
     "cs_check_finite": (_I32, [_VP, _I32, _P, _P]),
     "cs_check_positions": (_I32, [_P, _I64, _I32, _P, _P]),
+    "cs_check_inputs": (_I32, [_VP, ctypes.POINTER(_I32), _I32, _P, _I64, _P, _I64, _P, _P, _I32, _P]),
+    "cs_policy_lower": (_I32, [ctypes.POINTER(CsPolicyLowerArgs), _P]),
     "cs_check_bias_positions": (_I32, [_VP, _I64, _P, _P]),
     "cs_ccpe_attention": (_I32, [ctypes.POINTER(CsCcpeArgs), _P]),
     "cs_ccpe_attention_dense": (_I32, [ctypes.POINTER(CsCcpeArgs), _P]),

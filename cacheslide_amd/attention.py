@@ -11,6 +11,7 @@ calling them per query chunk:
 
 from __future__ import annotations
 
+import ctypes
 from dataclasses import dataclass, field
 
 import torch
@@ -102,9 +103,10 @@ def _policy_tables(policy: "CanonicalPositionPolicy", device) -> tuple:
 
 
 class _LoweredCanonical:
-    """Kernel inputs for one CanonicalPositionPolicy over one call's coordinates."""
+    """Kernel inputs for one CanonicalPositionPolicy over one call's coordinates
+    (``q_rows`` and ``k_ord`` are written by ``lower_policies``)."""
 
-    def __init__(self, policy: "CanonicalPositionPolicy", device, query_positions, key_positions):
+    def __init__(self, policy: "CanonicalPositionPolicy", device, nq: int, nk: int):
         # the call-independent part (position -> profile row / fixed ordinal
         # tables, the profile lookup's decision) once per profile, plan and
         # device: the runtime builds a new policy per call around the same
@@ -115,15 +117,9 @@ class _LoweredCanonical:
         hit = cache.get(key)
         if hit is None or hit[0] is not fixed:
             hit = cache[key] = (fixed, _policy_tables(policy, device))
-        q_dev, k_dev, size, self.unknown, self.profile_rows, self.fixed_count, self.reason = hit[1]
-        self.q_rows = torch.empty(query_positions.shape[0], dtype=torch.long, device=device)
-        self.k_ord = torch.empty(key_positions.shape[0], dtype=torch.long, device=device)
-        stream = _hip.stream_of(device)
-        call("cs_mapping_gather", ptr(q_dev), size, ptr(query_positions), ptr(self.q_rows),
-             query_positions.shape[0], stream)
-        call("cs_mapping_gather", ptr(k_dev), size, ptr(key_positions), ptr(self.k_ord),
-             key_positions.shape[0], stream)
-        self._tables = (q_dev, k_dev)
+        self.q_table, self.k_table, self.table_size, self.unknown, self.profile_rows, self.fixed_count, self.reason = hit[1]
+        self.q_rows = torch.empty(nq, dtype=torch.long, device=device)
+        self.k_ord = torch.empty(nk, dtype=torch.long, device=device)
         self.canonical = policy._canonical_on(device)
 
     def fits(self, heads: int) -> bool:
@@ -182,9 +178,6 @@ class CanonicalPositionPolicy:
             cache[key] = self.profile.canonical_positions.to(device)
         return cache[key]
 
-    def _lower(self, device, query_positions: Tensor, key_positions: Tensor) -> _LoweredCanonical:
-        return _LoweredCanonical(self, device, query_positions, key_positions)
-
     def __call__(self, contextual: Tensor, queries: Tensor, keys: Tensor) -> Tensor:
         """attention.py:32-57: substitute, then validate in strict mode."""
         ordinal = {position: i for i, position in enumerate(self.plan.fixed_indices)}
@@ -229,29 +222,18 @@ class SelectedAssociationPolicy:
     selected_indices: Tensor
 
     def _sets(self, device) -> tuple[Tensor, Tensor]:
-        """Fixed and selected positions on the device, each sorted ascending
-        (the kernels test membership by binary search)."""
+        """Fixed positions on the device, sorted ascending, and the selected ones
+        as given."""
         fixed_indices = self.fixed_indices
         if not isinstance(fixed_indices, tuple):
             fixed_indices = tuple(fixed_indices)
         fixed = _fixed_on(fixed_indices, device)
-        selected = self.selected_indices.to(device=device, dtype=torch.long).reshape(-1)
-        return fixed, torch.sort(selected).values
-
-    def _lower(self, device, query_positions: Tensor, key_positions: Tensor) -> tuple[Tensor, Tensor]:
-        fixed, selected = self._sets(device)
-        sel_rows = torch.empty(query_positions.shape[0], dtype=torch.uint8, device=device)
-        fixed_keys = torch.empty(key_positions.shape[0], dtype=torch.uint8, device=device)
-        stream = _hip.stream_of(device)
-        call("cs_isin", ptr(query_positions), query_positions.shape[0], ptr(selected),
-             selected.numel(), ptr(sel_rows), stream)
-        call("cs_isin", ptr(key_positions), key_positions.shape[0], ptr(fixed), fixed.numel(),
-             ptr(fixed_keys), stream)
-        return sel_rows, fixed_keys
+        return fixed, self.selected_indices.to(device=device, dtype=torch.long).reshape(-1).contiguous()
 
     def __call__(self, queries: Tensor, keys: Tensor) -> Tensor:
         device = _hip.require_device(queries, keys)
         fixed, selected = self._sets(device)
+        selected = torch.sort(selected).values
         nq, nk = queries.shape[0], keys.shape[0]
         buffer = torch.empty(nq * nk + nq + nk, dtype=torch.uint8, device=device)
         q = queries.to(torch.long).contiguous()
@@ -259,3 +241,28 @@ class SelectedAssociationPolicy:
         call("cs_selected_visibility", ptr(q), nq, ptr(k), nk, ptr(fixed), fixed.numel(),
              ptr(selected), selected.numel(), ptr(buffer), _hip.stream_of(device))
         return buffer[: nq * nk].view(torch.bool).view(nq, nk)
+
+
+def lower_policies(canonical: CanonicalPositionPolicy | None, selected: SelectedAssociationPolicy | None, device,
+                   query_positions: Tensor, key_positions: Tensor | None, nk: int):
+    """Kernel data of a call's policies in one launch: the lowered canonical
+    policy (or None) and the selected-row and fixed-key flags (or None, None).
+    ``key_positions`` None: keys at coordinates 0..nk-1."""
+    nq = query_positions.shape[0]
+    args = _hip.CsPolicyLowerArgs()
+    args.qpos, args.nq, args.nk = ptr(query_positions), nq, nk
+    args.kpos = ptr(key_positions)
+    lowered = sel_rows = fixed_keys = None
+    if canonical is not None:
+        lowered = _LoweredCanonical(canonical, device, nq, nk)
+        args.q_table, args.k_table, args.table_size = ptr(lowered.q_table), ptr(lowered.k_table), lowered.table_size
+        args.q_rows, args.k_ord = ptr(lowered.q_rows), ptr(lowered.k_ord)
+    if selected is not None:
+        fixed, chosen = selected._sets(device)
+        sel_rows = torch.empty(nq, dtype=torch.uint8, device=device)
+        fixed_keys = torch.empty(nk, dtype=torch.uint8, device=device)
+        args.fixed, args.n_fixed = ptr(fixed), fixed.numel()
+        args.selected, args.n_selected = ptr(chosen), chosen.numel()
+        args.sel_rows, args.fixed_keys = ptr(sel_rows), ptr(fixed_keys)
+    call("cs_policy_lower", ctypes.byref(args), _hip.stream_of(device))
+    return lowered, sel_rows, fixed_keys

@@ -111,12 +111,12 @@ def _kv_source(cache: Tensor, block_table: Tensor | None, slots: Tensor | None,
 
 def _prefill_dense(query: Tensor, key: Tensor, value: Tensor, e: Tensor,
                    query_positions: Tensor, ck) -> Tensor:
-    """One request, dense K/V [nk, Hkv, 128]; used by cope_attention's fast path."""
+    """One request, dense K/V [nk, Hkv, 128]; used by cope_attention's fast path
+    (``ck``'s scans have left the key count nk on the device)."""
     device = ck.device
     nq, hq = query.shape[0], query.shape[1]
     nk, hkv = key.shape[0], key.shape[1]
     out = torch.empty((1, nq, hq, 128), dtype=torch.bfloat16, device=device)
-    nk_dev = torch.full((1,), nk, dtype=torch.int32, device=device)
     src = _hip.CsKvSource()
     src.k, src.v = key.data_ptr(), value.data_ptr()
     src.k_s_batch, src.k_s_tok, src.k_s_head = 0, key.stride(0), key.stride(1)
@@ -126,7 +126,7 @@ def _prefill_dense(query: Tensor, key: Tensor, value: Tensor, e: Tensor,
         return _prefill_dense(q_c, k_c, v_c, e, query_positions, ck)
     call(
         "cs_ccpe_prefill_bf16", ptr(query), 0, query.stride(0), query.stride(1),
-        ptr(query_positions), 0, 1, nq, hq, hkv, ptr(nk_dev), src, ptr(e),
+        ptr(query_positions), 0, 1, nq, hq, hkv, ck.count_ptr, src, ptr(e),
         e.shape[1], ptr(out), ck.flags_ptr, ck.stream,
     )
     return out[0]

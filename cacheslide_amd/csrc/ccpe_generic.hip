@@ -348,11 +348,8 @@ __global__ void check_finite_kernel(dview v, int64_t numel, int32_t bit, int32_t
 // words (all-ones exponent = inf or NaN), four words in flight per thread.
 // KIND: 0 bf16, 1 f16, 2 f32, 3 f64.
 template <int KIND>
-__global__ void __launch_bounds__(256) check_finite_vec_kernel(const uint4* p, int64_t words,
-                                                               int32_t bit, int32_t* flags) {
+__device__ inline bool scan_words(const uint4* p, int64_t words, int64_t i, int64_t step) {
   bool bad = false;
-  const int64_t step = static_cast<int64_t>(gridDim.x) * blockDim.x;
-  int64_t i = blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x;
   for (; i + 3 * step < words; i += 4 * step) {
     uint4 v[4];
 #pragma unroll
@@ -361,6 +358,14 @@ __global__ void __launch_bounds__(256) check_finite_vec_kernel(const uint4* p, i
     for (int u = 0; u < 4; ++u) bad |= word_nonfinite<KIND>(v[u]);
   }
   for (; i < words; i += step) bad |= word_nonfinite<KIND>(p[i]);
+  return bad;
+}
+
+template <int KIND>
+__global__ void __launch_bounds__(256) check_finite_vec_kernel(const uint4* p, int64_t words,
+                                                               int32_t bit, int32_t* flags) {
+  const bool bad = scan_words<KIND>(p, words, blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x,
+                                    static_cast<int64_t>(gridDim.x) * blockDim.x);
   if (__any(bad) && (threadIdx.x & 63) == 0) atomicOr(flags, bit);
 }
 
@@ -391,6 +396,73 @@ __global__ void check_duplicates_kernel(const int64_t* pos, int64_t n, int32_t u
       if (pos[jdx] == p) { found = 1; break; }
   }
   if (__any(found) && (threadIdx.x & 63) == 0) atomicOr(flags, dup_bit);
+}
+
+// The input checks of one call in one launch: the finite scans of up to
+// kScans tensors (contiguous, in 16-byte words) and the order and duplicate
+// scans of up to two position lists.  Small calls wait for launches, not for
+// the scans: eight launches (three scans, two per list, and the list of
+// default key coordinates, which need no check) made a 211-token call 103 us,
+// this one makes it 68.
+constexpr int kScans = 3;
+constexpr int kScanLists = 2;
+constexpr int64_t kScanListMax = 32768;  // each block scans the whole list once
+struct check_inputs_params {
+  const uint4* data[kScans];
+  int64_t words[kScans];
+  int32_t kind[kScans], bit[kScans];
+  const int64_t* pos[kScanLists];
+  int32_t n[kScanLists], neg[kScanLists], uns[kScanLists], dup[kScanLists];
+  int32_t first[kScans + kScanLists + 1];  // first block of each part
+  int32_t* flags;
+  int32_t* count;  // receives count_value when non-null
+  int32_t count_value;
+};
+
+__global__ void __launch_bounds__(256) check_inputs_kernel(check_inputs_params a) {
+  const int blk = static_cast<int>(blockIdx.x), tid = threadIdx.x;
+  if (blk == 0 && tid == 0 && a.count) *a.count = a.count_value;
+#pragma unroll
+  for (int t = 0; t < kScans; ++t) {
+    if (blk < a.first[t] || blk >= a.first[t + 1]) continue;
+    const int64_t at = static_cast<int64_t>(blk - a.first[t]) * 256 + tid;
+    const int64_t step = static_cast<int64_t>(a.first[t + 1] - a.first[t]) * 256;
+    bool bad = false;
+    switch (a.kind[t]) {
+      case 0: bad = scan_words<0>(a.data[t], a.words[t], at, step); break;
+      case 1: bad = scan_words<1>(a.data[t], a.words[t], at, step); break;
+      case 2: bad = scan_words<2>(a.data[t], a.words[t], at, step); break;
+      default: bad = scan_words<3>(a.data[t], a.words[t], at, step); break;
+    }
+    if (__any(bad) && (tid & 63) == 0) atomicOr(a.flags, a.bit[t]);
+    return;
+  }
+#pragma unroll
+  for (int t = 0; t < kScanLists; ++t) {
+    if (blk < a.first[kScans + t] || blk >= a.first[kScans + t + 1]) continue;
+    // every block of a list scans its order: an ascending list has no
+    // duplicates, and otherwise each block looks for those of its own 256
+    const int64_t* pos = a.pos[t];
+    const int n = a.n[t];
+    int bits = 0;
+    for (int i = tid; i < n; i += 256) {
+      const int64_t p = pos[i];
+      if (p < 0) bits |= a.neg[t];
+      if (i > 0 && p <= pos[i - 1]) bits |= a.uns[t];
+    }
+    const bool unsorted = __syncthreads_or(bits & a.uns[t]) != 0;
+    if (unsorted) {
+      const int i = (blk - a.first[kScans + t]) * 256 + tid;
+      if (i < n) {
+        const int64_t p = pos[i];
+        for (int j = i + 1; j < n; ++j)
+          if (pos[j] == p) { bits |= a.dup[t]; break; }
+      }
+    }
+    for (int off = 32; off > 0; off >>= 1) bits |= __shfl_xor(bits, off, 64);
+    if (bits && (tid & 63) == 0) atomicOr(a.flags, bits);
+    return;
+  }
 }
 
 __global__ void check_bias_positions_kernel(dview v, int64_t numel, double top, int32_t* flags) {
@@ -474,17 +546,59 @@ __global__ void __launch_bounds__(64 * kGenWaves) positional_bias_kernel(
 }
 
 // Membership by binary search: `set` is sorted ascending.
-__global__ void isin_kernel(const int64_t* values, int64_t n, const int64_t* set, int64_t m,
-                            uint8_t* out) {
-  int64_t i = blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x;
-  if (i >= n) return;
-  const int64_t x = values[i];
+// Whether an ascending set holds x.
+__device__ inline bool sorted_contains(const int64_t* set, int64_t m, int64_t x) {
   int64_t lo = 0, hi = m;  // first element >= x
   while (lo < hi) {
     const int64_t mid = (lo + hi) >> 1;
     if (set[mid] < x) lo = mid + 1; else hi = mid;
   }
-  out[i] = (lo < m && set[lo] == x) ? 1 : 0;
+  return lo < m && set[lo] == x;
+}
+
+__global__ void isin_kernel(const int64_t* values, int64_t n, const int64_t* set, int64_t m,
+                            uint8_t* out) {
+  int64_t i = blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x;
+  if (i >= n) return;
+  out[i] = sorted_contains(set, m, values[i]) ? 1 : 0;
+}
+
+// The policy lowerings of one call in one launch: per query row its profile
+// row (q_table, -1 past its end) and whether it is selected, per key its fixed
+// ordinal (k_table) and whether it is fixed.  `fixed` is ascending; `selected`
+// is searched by halves when it is, as WCA's row lists are, else compared
+// value by value (no sort: a library sort of 2420 rows took 39 us, and six
+// launches).
+__global__ void __launch_bounds__(256) policy_lower_kernel(cs_policy_lower_args a) {
+  const int64_t q_blocks = (a.nq + 255) / 256;
+  const bool is_q = blockIdx.x < q_blocks;
+  const int64_t i = (is_q ? blockIdx.x : blockIdx.x - q_blocks) * 256 + threadIdx.x;
+  if (!is_q) {
+    if (i >= a.nk) return;
+    const int64_t j = a.kpos ? a.kpos[i] : i;
+    if (a.k_ord) a.k_ord[i] = j >= 0 && j < a.table_size ? a.k_table[j] : -1;
+    if (a.fixed_keys) a.fixed_keys[i] = sorted_contains(a.fixed, a.n_fixed, j) ? 1 : 0;
+    return;
+  }
+  const int64_t q = i < a.nq ? a.qpos[i] : -1;
+  if (a.q_rows && i < a.nq) a.q_rows[i] = q >= 0 && q < a.table_size ? a.q_table[q] : -1;
+  if (!a.sel_rows) return;
+  int descents = 0;
+  for (int64_t t = threadIdx.x + 1; t < a.n_selected; t += 256) descents |= a.selected[t] < a.selected[t - 1];
+  bool found = false;
+  if (__syncthreads_or(descents)) {
+    __shared__ int64_t part[256];
+    for (int64_t base = 0; base < a.n_selected; base += 256) {
+      const int n = static_cast<int>(a.n_selected - base < 256 ? a.n_selected - base : 256);
+      if (static_cast<int>(threadIdx.x) < n) part[threadIdx.x] = a.selected[base + threadIdx.x];
+      __syncthreads();
+      for (int t = 0; t < n; ++t) found = found || part[t] == q;
+      __syncthreads();
+    }
+  } else {
+    found = sorted_contains(a.selected, a.n_selected, q);
+  }
+  if (i < a.nq) a.sel_rows[i] = found ? 1 : 0;
 }
 
 __global__ void selected_visibility_kernel(const int64_t* queries, int64_t nq,
@@ -718,34 +832,49 @@ extern "C" int cs_ccpe_attention(const cs_ccpe_args* a, void* stream) {
   return CS_OK;
 }
 
-extern "C" int cs_check_finite(const cs_view* x, int32_t bit, int32_t* flags, void* stream) {
-  CS_REQUIRE(x && flags, "null arguments");
-  if (!x->data || !is_float_dtype(x->dtype)) return CS_OK;
-  int64_t numel = 1;
+namespace {
+
+// Whether a float view can be scanned in 16-byte words (contiguous, aligned,
+// whole words; or nothing to scan: words = 0), and how many.
+bool scan_layout(const cs_view* x, int64_t* words) {
+  *words = 0;
+  if (!x->data || !is_float_dtype(x->dtype)) return true;
+  int64_t numel = 1, expect = 1;
   for (int i = 0; i < x->ndim; ++i) numel *= x->shape[i];
-  if (numel == 0) return CS_OK;
-  bool contiguous = true;
-  int64_t expect = 1;
+  if (numel == 0) return true;
   for (int i = x->ndim - 1; i >= 0; --i) {
-    if (x->shape[i] != 1 && x->stride[i] != expect) contiguous = false;
+    if (x->shape[i] != 1 && x->stride[i] != expect) return false;
     expect *= x->shape[i];
   }
-  const int esize = dtype_size(x->dtype);
-  const int64_t bytes = numel * esize;
-  if (contiguous && (reinterpret_cast<uintptr_t>(x->data) & 15) == 0 && bytes % 16 == 0) {
-    const int64_t words = bytes / 16;
+  const int64_t bytes = numel * dtype_size(x->dtype);
+  if ((reinterpret_cast<uintptr_t>(x->data) & 15) != 0 || bytes % 16 != 0) return false;
+  *words = bytes / 16;
+  return true;
+}
+
+int finite_kind(int dtype) { return dtype == CS_BF16 ? 0 : dtype == CS_F16 ? 1 : dtype == CS_F32 ? 2 : 3; }
+
+}  // namespace
+
+extern "C" int cs_check_finite(const cs_view* x, int32_t bit, int32_t* flags, void* stream) {
+  CS_REQUIRE(x && flags, "null arguments");
+  int64_t words = 0;
+  if (scan_layout(x, &words)) {
+    if (words == 0) return CS_OK;
     const int grid = static_cast<int>(std::min<int64_t>(ceil_div(words, 256 * 4), 4096));
     const uint4* p = static_cast<const uint4*>(x->data);
     hipStream_t s = as_stream(stream);
-    switch (x->dtype) {
-      case CS_BF16: hipLaunchKernelGGL((check_finite_vec_kernel<0>), dim3(grid), dim3(256), 0, s, p, words, bit, flags); break;
-      case CS_F16: hipLaunchKernelGGL((check_finite_vec_kernel<1>), dim3(grid), dim3(256), 0, s, p, words, bit, flags); break;
-      case CS_F32: hipLaunchKernelGGL((check_finite_vec_kernel<2>), dim3(grid), dim3(256), 0, s, p, words, bit, flags); break;
+    switch (finite_kind(x->dtype)) {
+      case 0: hipLaunchKernelGGL((check_finite_vec_kernel<0>), dim3(grid), dim3(256), 0, s, p, words, bit, flags); break;
+      case 1: hipLaunchKernelGGL((check_finite_vec_kernel<1>), dim3(grid), dim3(256), 0, s, p, words, bit, flags); break;
+      case 2: hipLaunchKernelGGL((check_finite_vec_kernel<2>), dim3(grid), dim3(256), 0, s, p, words, bit, flags); break;
       default: hipLaunchKernelGGL((check_finite_vec_kernel<3>), dim3(grid), dim3(256), 0, s, p, words, bit, flags); break;
     }
     CS_LAUNCH_CHECK("check_finite");
     return CS_OK;
   }
+  int64_t numel = 1;
+  for (int i = 0; i < x->ndim; ++i) numel *= x->shape[i];
   dview v = to_dview(x);
   hipLaunchKernelGGL(check_finite_kernel, dim3(grid_for(numel, 256)), dim3(256), 0,
                      as_stream(stream), v, numel, bit, flags);
@@ -767,6 +896,57 @@ extern "C" int cs_check_positions(const int64_t* pos, int64_t n, int32_t is_key,
   hipLaunchKernelGGL(check_duplicates_kernel, dim3(grid_for(n, 256)), dim3(256), 0, s, pos, n, uns,
                      dup, flags);
   CS_LAUNCH_CHECK("check_positions");
+  return CS_OK;
+}
+
+extern "C" int cs_check_inputs(const cs_view* tensors, const int32_t* bits, int32_t n_tensors, const int64_t* qpos,
+                               int64_t nq, const int64_t* kpos, int64_t nk, int32_t* flags, int32_t* count,
+                               int32_t count_value, void* stream) {
+  CS_REQUIRE(flags && n_tensors >= 0 && (n_tensors == 0 || (tensors && bits)), "null arguments");
+  CS_REQUIRE(nq >= 0 && nk >= 0 && (nq == 0 || qpos) && (nk == 0 || kpos), "null positions");
+  check_inputs_params a{};
+  a.flags = flags;
+  a.count = count;
+  a.count_value = count_value;
+  int blocks = 0, used = 0;
+  for (int i = 0; i < n_tensors; ++i) {
+    const cs_view& x = tensors[i];
+    int64_t words = 0;
+    if (used == kScans || !scan_layout(&x, &words)) {
+      const int st = cs_check_finite(&x, bits[i], flags, stream);
+      if (st) return st;
+      continue;
+    }
+    if (words == 0) continue;
+    a.data[used] = static_cast<const uint4*>(x.data);
+    a.words[used] = words;
+    a.kind[used] = finite_kind(x.dtype);
+    a.bit[used] = bits[i];
+    a.first[used] = blocks;
+    blocks += static_cast<int>(std::min<int64_t>(ceil_div(words, 256 * 4), 2048));
+    ++used;
+  }
+  for (int t = used; t <= kScans; ++t) a.first[t] = blocks;
+  const int64_t* lists[kScanLists] = {qpos, kpos};
+  const int64_t sizes[kScanLists] = {nq, nk};
+  for (int t = 0; t < kScanLists; ++t) {
+    a.first[kScans + t] = blocks;
+    if (sizes[t] > kScanListMax) {
+      const int st = cs_check_positions(lists[t], sizes[t], t, flags, stream);
+      if (st) return st;
+    } else if (sizes[t] > 0) {
+      a.pos[t] = lists[t];
+      a.n[t] = static_cast<int32_t>(sizes[t]);
+      a.neg[t] = t ? CS_FLAG_KPOS_NEGATIVE : CS_FLAG_QPOS_NEGATIVE;
+      a.uns[t] = t ? CS_FLAG_KPOS_UNSORTED : kQposUnsortedInternal;
+      a.dup[t] = t ? CS_FLAG_KPOS_DUPLICATE : CS_FLAG_QPOS_DUPLICATE;
+      blocks += static_cast<int>(ceil_div(sizes[t], 256));
+    }
+  }
+  a.first[kScans + kScanLists] = blocks;
+  if (blocks == 0 && count == nullptr) return CS_OK;
+  hipLaunchKernelGGL(check_inputs_kernel, dim3(blocks > 0 ? blocks : 1), dim3(256), 0, as_stream(stream), a);
+  CS_LAUNCH_CHECK("check_inputs");
   return CS_OK;
 }
 
@@ -872,6 +1052,21 @@ extern "C" int cs_isin(const int64_t* values, int64_t n, const int64_t* set, int
   hipLaunchKernelGGL(isin_kernel, dim3(ceil_div(n, 256)), dim3(256), 0, as_stream(stream), values,
                      n, set, m, out);
   CS_LAUNCH_CHECK("isin");
+  return CS_OK;
+}
+
+extern "C" int cs_policy_lower(const cs_policy_lower_args* a, void* stream) {
+  CS_REQUIRE(a != nullptr && a->nq >= 0 && a->nk >= 0 && (a->nq == 0 || a->qpos), "null arguments");
+  CS_REQUIRE((a->q_rows != nullptr) == (a->k_ord != nullptr) || a->nq == 0 || a->nk == 0, "q_rows and k_ord go together");
+  CS_REQUIRE((!a->q_rows && !a->k_ord) || (a->q_table && a->k_table && a->table_size > 0), "null ordinal tables");
+  CS_REQUIRE(a->n_fixed >= 0 && a->n_selected >= 0 && (a->n_fixed == 0 || a->fixed) &&
+                 (a->n_selected == 0 || a->selected),
+             "null index lists");
+  const int64_t blocks = ceil_div(a->nq, 256) + ceil_div(a->nk, 256);
+  if (blocks == 0) return CS_OK;
+  CS_REQUIRE(blocks < (1ll << 31), "too many rows or keys");
+  hipLaunchKernelGGL(policy_lower_kernel, dim3(static_cast<uint32_t>(blocks)), dim3(256), 0, as_stream(stream), *a);
+  CS_LAUNCH_CHECK("policy_lower");
   return CS_OK;
 }
 

@@ -38,12 +38,28 @@ class CCPEPositionError(ValueError):
 # reference-ordered checks
 # --------------------------------------------------------------------------
 class _Checks:
-    """Host checks raise in order, after any earlier device check that failed."""
+    """Host checks raise in order, after any earlier device check that failed.
+
+    Scans of the inputs wait for ``launch_scans`` (or the first ``finish``)
+    and go out in one launch; word 1 of ``flags`` then holds ``count``."""
 
     def __init__(self, device: torch.device):
         self.device = device
-        self.flags = _hip.new_flags(device)
+        self.flags = _hip.new_flags(device, 2)
         self.steps: list[tuple[int, type, str]] = []
+        self.tensors: list[tuple[Tensor, int]] = []
+        self.lists: list[Tensor | None] = [None, None]  # query and key positions
+
+    def launch_scans(self, count: int | None = None) -> None:
+        tensors, self.tensors = self.tensors, []
+        (qpos, kpos), self.lists = self.lists, [None, None]
+        if not tensors and qpos is None and kpos is None and count is None:
+            return
+        views = (_hip.CsView * max(len(tensors), 1))(*(_hip.view(t) for t, _ in tensors))
+        bits = (ctypes.c_int32 * max(len(tensors), 1))(*(bit for _, bit in tensors))
+        call("cs_check_inputs", views, bits, len(tensors), ptr(qpos), 0 if qpos is None else qpos.shape[0], ptr(kpos),
+             0 if kpos is None else kpos.shape[0], self.flags_ptr, None if count is None else self.count_ptr,
+             count or 0, self.stream)
 
     def device_step(self, bits: int, exc: type, message: str) -> None:
         self.steps.append((bits, exc, message))
@@ -51,6 +67,7 @@ class _Checks:
     def finish(self, pending: BaseException | None = None, value: int | None = None) -> None:
         """Raise the first registered device check that fired, then ``pending``;
         ``value``: the flags word already read after the last launch."""
+        self.launch_scans()
         if value is None:
             value = _hip.read_flags(self.flags)[0] if self.steps else 0
         for bits, exc, message in self.steps:
@@ -67,6 +84,10 @@ class _Checks:
         return ptr(self.flags)
 
     @property
+    def count_ptr(self):
+        return ctypes.c_void_p(self.flags.data_ptr() + 4)
+
+    @property
     def stream(self):
         return _hip.stream_of(self.device)
 
@@ -78,7 +99,7 @@ def _device_of(tensor: Tensor) -> torch.device:
 
 
 def _finite_scan(ck: _Checks, tensor: Tensor, bit: int) -> None:
-    call("cs_check_finite", vref(tensor), bit, ck.flags_ptr, ck.stream)
+    ck.tensors.append((tensor, bit))
 
 
 def _rows(name: str, tensor: Tensor, ck: _Checks, bit: int) -> None:
@@ -110,7 +131,7 @@ def _positions(
         or tensor.device != device
     ):
         ck.fail(exc(f"{name} must be nonnegative int64 [{n}] on {device}"))
-    call("cs_check_positions", ptr(tensor), n, 1 if is_key else 0, ck.flags_ptr, ck.stream)
+    ck.lists[1 if is_key else 0] = tensor
     neg = _hip.FLAG_KPOS_NEGATIVE if is_key else _hip.FLAG_QPOS_NEGATIVE
     dup = _hip.FLAG_KPOS_DUPLICATE if is_key else _hip.FLAG_QPOS_DUPLICATE
     ck.device_step(neg, exc, f"{name} must be nonnegative int64 [{n}] on {device}")
@@ -517,7 +538,7 @@ def cope_attention(
     fused over all rows; any other callable is evaluated per query chunk on
     kernel-produced positions, as in the reference.
     """
-    from .attention import CanonicalPositionPolicy, SelectedAssociationPolicy
+    from .attention import CanonicalPositionPolicy, SelectedAssociationPolicy, lower_policies
 
     device = _device_of(query)
     ck = _Checks(device)
@@ -539,10 +560,9 @@ def cope_attention(
             ck.fail(ValueError("visibility_transform and visibility_mask are mutually exclusive"))
     nq, hq, nk = query.shape[0], query.shape[1], key.shape[0]
     _positions("query_positions", query_positions, nq, device, ck, False)
-    default_keys = key_positions is None
-    if default_keys:
-        key_positions = torch.arange(nk, device=device)
-    _positions("key_positions", key_positions, nk, device, ck, True)
+    default_keys = key_positions is None   # coordinates 0..nk-1: nothing to check
+    if not default_keys:
+        _positions("key_positions", key_positions, nk, device, ck, True)
     for name, mask in (("attention_mask", attention_mask), ("visibility_mask", visibility_mask)):
         if mask is not None and mask.shape not in ((nq, nk), (1, nq, nk), (hq, nq, nk)):
             ck.fail(ValueError(f"{name} has an incompatible full-query shape"))
@@ -566,6 +586,9 @@ def cope_attention(
     selected = visibility_transform if isinstance(visibility_transform, SelectedAssociationPolicy) else None
     generic_positions = positions_transform is not None and canonical is None
     generic_visibility = visibility_transform is not None and selected is None
+    ck.launch_scans(count=nk)
+    if default_keys and (generic_positions or generic_visibility):
+        key_positions = torch.arange(nk, device=device)
     if generic_positions or generic_visibility:
         return _chunked_attention(
             query, key, value, cope, query_positions, key_positions, amask, visibility_mask,
@@ -596,8 +619,11 @@ def cope_attention(
             return output
         # values near or past the end of the finite range: the generic kernel
         # decides between the result and the reference's error
-        ck.flags.bitwise_and_(~_hip.FLAG_POLICY_GENERIC)
+        ck.flags[:1].bitwise_and_(~_hip.FLAG_POLICY_GENERIC)
 
+    policy = canonical is not None or selected is not None
+    if default_keys and not policy:
+        key_positions = torch.arange(nk, device=device)
     if fixed_positions is not None:
         call("cs_check_bias_positions", vref(fixed_positions), cope.max_positions, ck.flags_ptr, ck.stream)
 
@@ -615,8 +641,10 @@ def cope_attention(
     keep = []
     chunk_flags = None
     lowered = None
+    sel_rows = fixed_keys = None
+    if policy:
+        lowered, sel_rows, fixed_keys = lower_policies(canonical, selected, device, query_positions, key_positions, nk)
     if canonical is not None:
-        lowered = canonical._lower(device, query_positions, key_positions)
         if lowered.reason or not lowered.fits(hq):
             # A profile that does not match the plan is only an error when some
             # query row is fixed; it is never handed to the kernel.
@@ -639,7 +667,6 @@ def cope_attention(
         args.chunk_rows = query_chunk_size
         args.chunk_flags = ptr(chunk_flags)
     if selected is not None:
-        sel_rows, fixed_keys = selected._lower(device, query_positions, key_positions)
         keep += [sel_rows, fixed_keys]
         args.sel_rows = ptr(sel_rows)
         args.fixed_keys = ptr(fixed_keys)
@@ -649,12 +676,12 @@ def cope_attention(
     # for the device per call).
     flags_value = None
     chunk_values = None
-    if ((selected is not None or canonical is not None) and default_keys
+    if (policy and default_keys
             and _policy_fast_ok(query, key, value, e, cope, amask, visibility_mask, fixed_positions,
                                 return_positions, lowered if canonical is not None else None)
             and _policy_prefill(args, query, key, ck)):
         if chunk_flags is not None:
-            chunk_buf[n_chunks:].copy_(ck.flags)
+            chunk_buf[n_chunks:].copy_(ck.flags[:1])
             values = _hip.read_flags(chunk_buf)
             flags_value, chunk_values = values[-1], values[:-1]
         else:
@@ -662,14 +689,14 @@ def cope_attention(
         if flags_value & _hip.FLAG_POLICY_GENERIC:
             # more fixed/dynamic boundary keys than the path checker holds: the
             # generic kernel runs the call
-            ck.flags.bitwise_and_(~_hip.FLAG_POLICY_GENERIC)
+            ck.flags[:1].bitwise_and_(~_hip.FLAG_POLICY_GENERIC)
             if chunk_flags is not None:
                 chunk_flags.zero_()
             flags_value = None
             chunk_values = None
-            call("cs_ccpe_attention", args, ck.stream)
+            _generic_attention(args, key_positions, nk, ck)
     else:
-        call("cs_ccpe_attention", args, ck.stream)
+        _generic_attention(args, key_positions, nk, ck)
     ck.device_step(_hip.FLAG_LOGIT_NONFINITE, ValueError, "attention logits overflowed the accumulation dtype")
     ck.device_step(_hip.FLAG_POS_INVALID, ValueError, "positions must be bounded query-dependent [head,query,key]")
     ck.device_step(_hip.FLAG_SCORE_NONFINITE, ValueError, "contextual attention logits are not finite")
@@ -679,6 +706,14 @@ def cope_attention(
     if return_positions:
         return output, trace
     return output
+
+
+def _generic_attention(args, key_positions: Tensor | None, nk: int, ck: _Checks) -> None:
+    """cs_ccpe_attention, which takes the key coordinates as a list."""
+    if key_positions is None:
+        key_positions = torch.arange(nk, device=ck.device)
+        args.kpos = ptr(key_positions)
+    call("cs_ccpe_attention", args, ck.stream)
 
 
 _TRANSFORM_BOUNDS_MESSAGE = ("positions_transform must return bounded finite positions "

@@ -107,6 +107,14 @@ int cs_check_finite(const cs_view* x, int32_t bit, int32_t* flags, void* stream)
 int cs_check_positions(const int64_t* pos, int64_t n, int32_t is_key,
                        int32_t* flags, void* stream);
 
+/* cs_check_finite of each of n_tensors views (bit bits[i]) and
+ * cs_check_positions of the query list (and, when nk > 0, of the key list) in
+ * one launch where the layouts allow.  count (may be null) receives
+ * count_value on the device. */
+int cs_check_inputs(const cs_view* tensors, const int32_t* bits, int32_t n_tensors, const int64_t* qpos,
+                    int64_t nq, const int64_t* kpos, int64_t nk, int32_t* flags, int32_t* count,
+                    int32_t count_value, void* stream);
+
 /* Positions tensor [H, q, k] used as CoPE coordinates: ORs CS_FLAG_POS_INVALID
  * when an entry is nonfinite, < 0 or > max_positions-1 (position.py:323-334,
  * 504-516), and CS_FLAG_POS_NONFINITE when an entry is nonfinite. */
@@ -244,6 +252,32 @@ int cs_selected_visibility(const int64_t* queries, int64_t nq, const int64_t* ke
  * SelectedAssociationPolicy, attention.py:60-72); set sorted ascending. */
 int cs_isin(const int64_t* values, int64_t n, const int64_t* set, int64_t m, uint8_t* out,
             void* stream);
+
+/* The kernel data of both policies of one call (attention.py:18-72), in one
+ * launch.  kpos null: keys at coordinates 0..nk-1.  CanonicalPositionPolicy
+ * (q_rows and k_ord, or neither): q_rows[i] = q_table[qpos[i]], k_ord[j] =
+ * k_table[kpos[j]], -1 past the tables' table_size entries.
+ * SelectedAssociationPolicy (sel_rows, fixed_keys; each may be null):
+ * membership of qpos[i] in `selected` (any order) and of kpos[j] in `fixed`
+ * (ascending). */
+typedef struct cs_policy_lower_args {
+  const int64_t* qpos;
+  int64_t nq;
+  const int64_t* kpos;
+  int64_t nk;
+  const int64_t* q_table;
+  const int64_t* k_table;
+  int64_t table_size;
+  int64_t* q_rows;
+  int64_t* k_ord;
+  const int64_t* fixed;
+  int64_t n_fixed;
+  const int64_t* selected;
+  int64_t n_selected;
+  uint8_t* sel_rows;
+  uint8_t* fixed_keys;
+} cs_policy_lower_args;
+int cs_policy_lower(const cs_policy_lower_args* args, void* stream);
 
 /* CanonicalPositionPolicy substitution (attention.py:46-50):
  * result[h, rows[i], cols[c]] = canonical[h, q_ord_rows[i], k_ord_cols[c]]. */
