@@ -143,6 +143,19 @@ class CsPolicyLowerArgs(ctypes.Structure):
                              "fixed", "n_fixed", "selected", "n_selected", "sel_rows", "fixed_keys")]
 
 
+class CsDecoderLayerArgs(ctypes.Structure):
+    """cs_decoder_layer_args: one decoder layer around its attention call."""
+
+    _fields_ = (
+        [(name, ctypes.c_int32) for name in ("batch", "hidden", "heads", "kv_heads", "ffn")]
+        + [("eps", ctypes.c_float)]
+        + [(name, ctypes.c_void_p) for name in ("qkv", "o", "gate_up", "down", "in_norm", "post_norm", "residual", "q",
+                                                "attn", "act", "cache")]
+        + [(name, ctypes.c_int64) for name in ("s_block", "s_head", "s_offset", "blocks")]
+        + [("block_size", ctypes.c_int32), ("table", ctypes.c_void_p), ("table_stride", ctypes.c_int64),
+           ("table_cols", ctypes.c_int64), ("positions", ctypes.c_void_p), ("flags", ctypes.c_void_p)])
+
+
 class CsKvSource(ctypes.Structure):
     _fields_ = [
         ("cache", ctypes.c_void_p),
@@ -247,6 +260,10 @@ SIGNATURES = {
         [_P, _I64, _I64, _I32, _I32, _I32, _P, _I32, ctypes.POINTER(CsKvSource), _P,
          _I32, _I32, _P, _P, _P],
     ),
+    "cs_decoder_qkv": (_I32, [ctypes.POINTER(CsDecoderLayerArgs), _P]),
+    "cs_decoder_mlp": (_I32, [ctypes.POINTER(CsDecoderLayerArgs), _P]),
+    "cs_decoder_context": (_I32, [_P, _I32, _P, _P]),
+    "cs_decoder_head": (_I32, [_P, _P, _P, _P, _I32, _I32, _I32, ctypes.c_float, _P]),
     "cs_slot_scatter": (_I32, [_VP, _VP, _VP, _P, _P, _I64, _VP, _VP, _P]),
     "cs_slot_gather": (_I32, [_VP, _VP, _VP, _P, _P, _I64, _VP, _VP, _P]),
     "cs_slot_copy": (_I32, [_VP, _P, _P, _I64, _P]),

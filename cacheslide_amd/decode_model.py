@@ -15,7 +15,9 @@ once at the end.
 
 All layers share one block table (one paged cache tensor per layer, the vLLM
 layout [blocks, KV heads, block_size, 2 x 128]).  Weights are bf16 from
-``torch.Generator`` seeds; the projections are plain library GEMMs.
+``torch.Generator`` seeds; the projections are plain library GEMMs, or for a
+few requests kernels that stream the weights once with the rest of the layer
+fused into them (``cs_decoder_*``).
 """
 
 from __future__ import annotations
@@ -27,11 +29,13 @@ import torch.nn.functional as F
 from torch import Tensor
 
 from . import _hip
+from ._hip import call, ptr
 from .ccpe import (SharedRuns, ccpe_decode_paged, ccpe_decode_shared, decode_shared_workspace, decode_workspace,
                    raise_flags)
 from .position import CoPE
 
 HEAD_DIM = 128
+FUSED_BATCH = 32   # requests up to which a step's projections are cs_decoder_* launches
 
 
 @dataclass(frozen=True)
@@ -125,6 +129,9 @@ class PagedDecoder:
         s = self.shape
         b = ids.shape[0]
         bs = caches[0].shape[2]
+        if 1 <= b <= FUSED_BATCH and self._fused_ok(ids, positions, caches, block_table, flags, attn_out):
+            return self._step_fused(ids, positions, caches, block_table, max_context, workspace, flags, split,
+                                    attn_out, shared)
         slots = block_table.gather(1, (positions // bs).unsqueeze(1)).squeeze(1).long() * bs + positions % bs
         context = (positions + 1).to(torch.int32)
         if attn_out is None:
@@ -160,6 +167,75 @@ class PagedDecoder:
             gate, up = (h @ layer.gate_up.T).split(s.ffn, dim=-1)
             x = (F.silu(gate) * up) @ layer.down.T
         return self._rms(x + residual, self.norm) @ self.lm_head.T
+
+    def _fused_ok(self, ids, positions, caches, block_table, flags, attn_out) -> bool:
+        """Whether the layout is the one cs_decoder_* reads: bf16 weights as
+        built, contiguous int64 ids and positions, bf16 caches with whole
+        contiguous records."""
+        s = self.shape
+
+        def plain(t, dtype, *dims):
+            return t.dtype == dtype and t.shape == dims and t.is_contiguous() and t.device == caches[0].device
+
+        wide = (s.heads + 2 * s.kv_heads) * HEAD_DIM
+        bf16, b = torch.bfloat16, ids.shape[0]
+        return (
+            s.ffn % 32 == 0 and len(caches) == len(self.layers) and plain(positions, torch.long, b)
+            and ids.dtype == torch.long and ids.ndim == 1
+            and block_table.dtype == torch.int32 and block_table.ndim == 2 and block_table.stride(1) == 1
+            and block_table.shape[0] == b and block_table.shape[1] > 0 and block_table.device == caches[0].device
+            and flags.dtype == torch.int32 and flags.numel() >= 1 and flags.device == caches[0].device
+            and (attn_out is None or plain(attn_out, bf16, b, s.heads, HEAD_DIM))
+            and plain(self.embed, bf16, s.vocab, s.hidden) and plain(self.lm_head, bf16, s.vocab, s.hidden)
+            and plain(self.norm, bf16, s.hidden)
+            and all(c.dtype == bf16 and c.ndim == 4 and c.shape[1:] == caches[0].shape[1:]
+                    and c.shape[1] == s.kv_heads and c.shape[3] == 2 * HEAD_DIM and c.stride(3) == 1
+                    and c.data_ptr() % 16 == 0 for c in caches)
+            and all(plain(layer.qkv, bf16, wide, s.hidden) and plain(layer.o, bf16, s.hidden, s.hidden)
+                    and plain(layer.gate_up, bf16, 2 * s.ffn, s.hidden) and plain(layer.down, bf16, s.hidden, s.ffn)
+                    and plain(layer.in_norm, bf16, s.hidden) and plain(layer.post_norm, bf16, s.hidden)
+                    for layer in self.layers))
+
+    def _step_fused(self, ids, positions, caches, block_table, max_context, workspace, flags, split, attn_out,
+                    shared) -> Tensor:
+        """``step`` with each layer's launches fused around its attention call
+        (cs_decoder_qkv, cs_decoder_mlp)."""
+        s, b = self.shape, ids.shape[0]
+        stream = _hip.stream_of(self.device)
+        residual = self.embed[ids]
+        context = torch.empty(b, dtype=torch.int32, device=residual.device)
+        call("cs_decoder_context", ptr(positions), b, ptr(context), stream)
+        rows = torch.empty((2, b, s.heads, HEAD_DIM), dtype=self.dtype, device=residual.device)
+        q = rows[0]
+        if attn_out is None:
+            attn_out = rows[1]
+        act = torch.empty((b, s.ffn), dtype=self.dtype, device=residual.device)
+        tail = shared.tail_lens(context) if shared is not None else None
+        args = _hip.CsDecoderLayerArgs()
+        args.batch, args.hidden, args.heads, args.kv_heads, args.ffn = b, s.hidden, s.heads, s.kv_heads, s.ffn
+        args.eps = s.eps
+        args.residual, args.q, args.attn, args.act = (t.data_ptr() for t in (residual, q, attn_out, act))
+        args.table, args.table_stride, args.table_cols = block_table.data_ptr(), block_table.stride(0), block_table.shape[1]
+        args.positions, args.flags = positions.data_ptr(), flags.data_ptr()
+        for layer, cache in zip(self.layers, caches):
+            args.qkv, args.o = layer.qkv.data_ptr(), layer.o.data_ptr()
+            args.gate_up, args.down = layer.gate_up.data_ptr(), layer.down.data_ptr()
+            args.in_norm, args.post_norm = layer.in_norm.data_ptr(), layer.post_norm.data_ptr()
+            args.cache, args.blocks, args.block_size = cache.data_ptr(), cache.shape[0], cache.shape[2]
+            args.s_block, args.s_head, args.s_offset = cache.stride()[:3]
+            call("cs_decoder_qkv", args, stream)
+            if shared is not None:
+                ccpe_decode_shared(q, cache, block_table, context, layer.cope, shared, max_context=max_context,
+                                   split=split, tail=tail, workspace=workspace, out=attn_out, flags=flags,
+                                   check=False)
+            else:
+                ccpe_decode_paged(q, cache, block_table, context, layer.cope, max_context=max_context,
+                                  split=split, workspace=workspace, out=attn_out, flags=flags, check=False)
+            call("cs_decoder_mlp", args, stream)
+        logits = torch.empty((b, s.vocab), dtype=self.dtype, device=residual.device)
+        call("cs_decoder_head", ptr(residual), ptr(self.norm), ptr(self.lm_head), ptr(logits), b, s.hidden, s.vocab,
+             s.eps, stream)
+        return logits
 
     def generate(self, first_ids: Tensor, lengths: Tensor, caches: list[Tensor], block_table: Tensor,
                  steps: int, *, max_context: int, split: int = 1024, check: bool = True,

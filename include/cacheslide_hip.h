@@ -435,6 +435,43 @@ int cs_ccpe_decode_bf16_noalloc(const void* q, int64_t q_s_batch, int64_t q_s_he
                                 int32_t max_positions, int32_t split, void* out, int32_t* flags,
                                 void* stream);
 
+/* One decoder layer of a token of each of at most 32 requests around its
+ * attention call (reference.py:177-193), all bf16: cs_decoder_qkv writes the
+ * q rows [B, heads x 128] of the normed residual rows and the new K/V records
+ * to block table[b, p / bs], offset p % bs of each request's position p (a
+ * record outside the table or the cache is skipped and sets
+ * CS_FLAG_BLOCK_INVALID); cs_decoder_mlp adds the output projection of `attn`
+ * and then the gated MLP to the residual rows, in place.  Weights [out, in]
+ * contiguous, 16-byte aligned; hidden = heads x 128; ffn a multiple of 32. */
+typedef struct cs_decoder_layer_args {
+  int32_t batch, hidden, heads, kv_heads, ffn;
+  float eps;
+  const void* qkv;       /* [(heads + 2 kv_heads) x 128, hidden] */
+  const void* o;         /* [hidden, hidden] */
+  const void* gate_up;   /* [2 ffn, hidden]: gate rows, then up rows */
+  const void* down;      /* [hidden, ffn] */
+  const void* in_norm;   /* [hidden] */
+  const void* post_norm; /* [hidden] */
+  void* residual;        /* [B, hidden] */
+  void* q;               /* [B, heads x 128] */
+  const void* attn;      /* [B, heads x 128] */
+  void* act;             /* [B, ffn] scratch */
+  void* cache;           /* [blocks, kv_heads, block_size, 256], element strides below */
+  int64_t s_block, s_head, s_offset, blocks;
+  int32_t block_size;
+  const int32_t* table;  /* [B, table_cols] */
+  int64_t table_stride, table_cols;
+  const int64_t* positions; /* [B] */
+  int32_t* flags;
+} cs_decoder_layer_args;
+int cs_decoder_qkv(const cs_decoder_layer_args* args, void* stream);
+int cs_decoder_mlp(const cs_decoder_layer_args* args, void* stream);
+/* out[i] = positions[i] + 1: the key counts of a step's attention calls. */
+int cs_decoder_context(const int64_t* positions, int32_t n, int32_t* out, void* stream);
+/* Logits [B, vocab] of the final norm and the LM head w [vocab, hidden]. */
+int cs_decoder_head(const void* x, const void* norm, const void* w, void* out, int32_t batch, int32_t hidden,
+                    int32_t vocab, float eps, void* stream);
+
 /* ------------------------------------------------------------------------ *
  * SLIDE slot kernels (paged.py:205-240, 433-472; slide.py:103-112).
  * cache [blocks, H, bs, 2D] any dtype; side_k/side_v [S, H, D] (may be absent).
