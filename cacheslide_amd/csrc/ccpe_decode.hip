@@ -1388,25 +1388,23 @@ extern "C" int cs_ccpe_decode_shared_bf16(const cs_decode_shared_args* a, void* 
                                    a->split);
   hipStream_t s = as_stream(stream);
   // head: every run once for all requests (rows = requests), positions P-1
-  if (a->head_items > 0) {
-    cs_kv_source kh = *a->kv;
-    kh.block_table = a->head_table;
-    kh.bt_stride = a->head_blocks;
-    kh.bt_cols = a->head_blocks;
-    st = cs::launch_prefill_states(a->q, 0, a->q_s_batch, a->q_s_head, a->head_qpos, a->batch, a->head_items,
-                                   a->batch, a->hq, a->hkv, a->head_nk, &kh, a->e, a->max_positions, 1, 8,
-                                   w.head_o, w.head_ml, nullptr, a->flags, s);
-    if (st) return st;
-  }
+  cs_kv_source kh = *a->kv;
+  kh.block_table = a->head_table;
+  kh.bt_stride = a->head_blocks;
+  kh.bt_cols = a->head_blocks;
+  const cs::prefill_states_call head{a->q, 0, a->q_s_batch, a->q_s_head, a->head_qpos, a->batch, a->head_items,
+                                     a->batch, a->hq, a->hkv, a->head_nk, &kh, a->e, a->max_positions, 1, 8,
+                                     w.head_o, w.head_ml, nullptr, a->flags};
   // tail: one query row per request, exact positions, narrow workgroups;
-  // the launch also clears the fallback's gate word
+  // it also clears the fallback's gate word
   cs_kv_source kt = *a->kv;
   kt.block_table = a->tail_table;
   kt.bt_stride = a->tail_stride;
   kt.bt_cols = a->tail_cols;
-  st = cs::launch_prefill_states(a->q, a->q_s_batch, 0, a->q_s_head, a->tail_qpos, 1, a->batch, 1, a->hq, a->hkv,
-                                 a->tail_nk, &kt, a->e, a->max_positions, 0, 2, w.tail_o, w.tail_ml, w.gate,
-                                 a->flags, s);
+  const cs::prefill_states_call tail{a->q, a->q_s_batch, 0, a->q_s_head, a->tail_qpos, 1, a->batch, 1, a->hq,
+                                     a->hkv, a->tail_nk, &kt, a->e, a->max_positions, 0, 2, w.tail_o, w.tail_ml,
+                                     w.gate, a->flags};
+  st = cs::launch_prefill_states_pair(head, tail, s);
   if (st) return st;
   const int group = a->hq / a->hkv;
   hipLaunchKernelGGL(shared_merge_kernel, dim3(static_cast<uint32_t>(a->batch) * a->hkv), dim3(kD * group), 0, s,

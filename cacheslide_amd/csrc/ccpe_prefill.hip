@@ -73,8 +73,8 @@ constexpr size_t kStaticLds = kStages * 2 * kStageSlots * 16 + 4 * kBtWindow + 1
 // own, at its canonical position; a fixed row that is not selected sees every
 // fixed key at its canonical position (the calibration-layer call, and
 // selected_attention "all"); other rows keep their contextual positions.
-template <int MODE, int WAVES, bool POLICY = false>
-__global__ void __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(2, 2))) ccpe_prefill_kernel(prefill_params p) {
+template <int MODE, int WAVES, bool POLICY>
+__device__ __forceinline__ void prefill_workgroup(const prefill_params& p, const int wg_id) {
   constexpr bool PAGED = MODE != 0;
   constexpr bool SLOTS = MODE == 2;
   constexpr int kThreads = 64 * WAVES;
@@ -103,17 +103,17 @@ __global__ void __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu
   // saturated.  Each part leaves its softmax state in slot slot0 + part.
   int part = 0, nparts = 1, slot0 = 0, t_split = 0;
   if (!POLICY || p.split_role == 0) {
-    decode_wg(p, b, kvh, rb);
+    decode_wg(p, wg_id, b, kvh, rb);
   } else {
     int logical;
     if (p.split_role == 1) {
-      if (static_cast<int>(blockIdx.x) < p.split_extra) {
-        const int32_t item = uniform_load(p.split_items, static_cast<int64_t>(blockIdx.x));
+      if (wg_id < p.split_extra) {
+        const int32_t item = uniform_load(p.split_items, static_cast<int64_t>(wg_id));
         if (item < 0) return;  // an unused extra part: the whole workgroup, before any barrier
         logical = item >> 4;
         part = item & 15;
       } else {
-        logical = logical_wg(p, static_cast<int>(blockIdx.x) - p.split_extra);
+        logical = logical_wg(p, wg_id - p.split_extra);
       }
       nparts = uniform_load(p.split_plan, 3 * static_cast<int64_t>(logical));
       slot0 = uniform_load(p.split_plan, 3 * static_cast<int64_t>(logical) + 1);
@@ -122,7 +122,7 @@ __global__ void __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu
       // fix-up: a split block whose part 0 left some column's positions below
       // P-1 (its other parts then took unsaturated keys as saturated) is
       // walked again unsplit; every other workgroup ends here
-      logical = uniform_load(p.split_blocks, static_cast<int64_t>(blockIdx.x));
+      logical = uniform_load(p.split_blocks, static_cast<int64_t>(wg_id));
       if (logical < 0) return;
       const int s0 = uniform_load(p.split_plan, 3 * static_cast<int64_t>(logical) + 1);
       const float* carries = p.part_ml + (static_cast<int64_t>(s0) * 3 + 2) * 256;
@@ -183,7 +183,7 @@ __global__ void __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu
   }
 
   if (tid == 0) wg_max_pos = 0;
-  if (tid == 0 && blockIdx.x == 0 && p.zero_word != nullptr) *p.zero_word = 0;
+  if (tid == 0 && wg_id == 0 && p.zero_word != nullptr) *p.zero_word = 0;
   __syncthreads();
   int64_t wmax = qp, wmin = row_ok ? qp : INT64_MAX;
   for (int off = 32; off > 0; off >>= 1) {
@@ -904,6 +904,24 @@ walk_done:
   if (bad_block) atomicOr(p.flags, CS_FLAG_BLOCK_INVALID);
 }
 
+template <int MODE, int WAVES, bool POLICY = false>
+__global__ void __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(2, 2))) ccpe_prefill_kernel(prefill_params p) {
+  prefill_workgroup<MODE, WAVES, POLICY>(p, static_cast<int>(blockIdx.x));
+}
+
+// Two block-table calls in one launch: workgroups [0, a.total_wg) run `a`, the
+// others `b`.  For calls that each leave the chip half empty (the runs and the
+// tails of a shared-run decode).
+template <int WAVES>
+__global__ void __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(2, 2)))
+ccpe_prefill_pair_kernel(prefill_params a, prefill_params b) {
+  const int id = static_cast<int>(blockIdx.x);
+  if (id < a.total_wg)
+    prefill_workgroup<1, WAVES, false>(a, id);
+  else
+    prefill_workgroup<1, WAVES, false>(b, id - a.total_wg);
+}
+
 }  // namespace
 }  // namespace cs
 
@@ -1507,30 +1525,26 @@ extern "C" int cs_ccpe_prefill_bf16(const void* q, int64_t q_s_batch, int64_t q_
 
 namespace cs {
 
-// The paged MFMA prefill writing softmax states (state_o, state_ml: see
-// prefill_params) instead of output rows; saturated: every position taken as
-// P-1; zero_word (may be null) is set to 0.  Workgroups of at most max_waves
-// wavefronts.
-int launch_prefill_states(const void* q, int64_t q_s_batch, int64_t q_s_tok, int64_t q_s_head,
-                          const int64_t* qpos, int64_t qpos_s_batch, int32_t batch, int32_t nq, int32_t hq,
-                          int32_t hkv, const int32_t* nk, const cs_kv_source* kv, const float* e,
-                          int32_t max_positions, int32_t saturated, int max_waves, float* state_o,
-                          float* state_ml, int32_t* zero_word, int32_t* flags, hipStream_t s) {
-  CS_REQUIRE(state_o && state_ml, "null state buffers");
-  cs::prefill_params p{};
-  int waves = 4;
-  size_t smem = 0;
-  const int st = prepare_prefill(q, q_s_batch, q_s_tok, q_s_head, qpos, qpos_s_batch, batch, nq, hq, hkv, nk, kv,
-                                 e, max_positions, state_o, flags, &p, &waves, &smem, max_waves);
+namespace {
+
+// A block-table call writing softmax states (state_o, state_ml: see
+// prefill_params) instead of output rows.
+int prepare_states(const prefill_states_call& c, cs::prefill_params* p, int* waves, size_t* smem) {
+  CS_REQUIRE(c.state_o && c.state_ml, "null state buffers");
+  const int st = prepare_prefill(c.q, c.q_s_batch, c.q_s_tok, c.q_s_head, c.qpos, c.qpos_s_batch, c.batch, c.nq, c.hq,
+                                 c.hkv, c.nk, c.kv, c.e, c.max_positions, c.state_o, c.flags, p, waves, smem,
+                                 c.max_waves);
   if (st) return st;
-  if (batch == 0 || nq == 0) return CS_OK;
-  p.state_o = state_o;
-  p.state_ml = state_ml;
-  p.saturated = saturated ? 1 : 0;
-  p.zero_word = zero_word;
+  CS_REQUIRE(p->kv.block_table && !p->kv.slots, "softmax states are written for block-table calls only");
+  p->state_o = c.state_o;
+  p->state_ml = c.state_ml;
+  p->saturated = c.saturated ? 1 : 0;
+  p->zero_word = c.zero_word;
+  return CS_OK;
+}
+
+int launch_states(const cs::prefill_params& p, int waves, size_t smem, hipStream_t s) {
   const dim3 grid(p.total_wg), block(64 * waves);
-  const int mode = p.kv.slots ? 2 : (p.kv.block_table ? 1 : 0);
-  CS_REQUIRE(mode == 1, "softmax states are written for block-table calls only");
   if (waves == 8)
     hipLaunchKernelGGL((ccpe_prefill_kernel<1, 8>), grid, block, smem, s, p);
   else if (waves == 2)
@@ -1538,6 +1552,36 @@ int launch_prefill_states(const void* q, int64_t q_s_batch, int64_t q_s_tok, int
   else
     hipLaunchKernelGGL((ccpe_prefill_kernel<1, 4>), grid, block, smem, s, p);
   CS_LAUNCH_CHECK("ccpe_prefill_states");
+  return CS_OK;
+}
+
+}  // namespace
+
+// Two calls that write softmax states; either may have no rows.  One launch
+// when both run 2-wave workgroups and do not fill the chip (at 32 requests over
+// eight 1024-token runs: 25 and 20 us one after the other, 30 us together).
+int launch_prefill_states_pair(const prefill_states_call& first, const prefill_states_call& second, hipStream_t s) {
+  cs::prefill_params p[2];
+  int waves[2] = {0, 0};
+  size_t smem[2] = {0, 0};
+  const prefill_states_call* calls[2] = {&first, &second};
+  for (int i = 0; i < 2; ++i) {
+    if (calls[i]->batch == 0 || calls[i]->nq == 0) continue;
+    const int st = prepare_states(*calls[i], &p[i], &waves[i], &smem[i]);
+    if (st) return st;
+  }
+  const int64_t total = static_cast<int64_t>(waves[0] ? p[0].total_wg : 0) + (waves[1] ? p[1].total_wg : 0);
+  if (waves[0] == 2 && waves[1] == 2 && total < (1ll << 31)) {
+    hipLaunchKernelGGL((ccpe_prefill_pair_kernel<2>), dim3(static_cast<uint32_t>(total)), dim3(128),
+                       smem[0] > smem[1] ? smem[0] : smem[1], s, p[0], p[1]);
+    CS_LAUNCH_CHECK("ccpe_prefill_pair");
+    return CS_OK;
+  }
+  for (int i = 0; i < 2; ++i) {
+    if (waves[i] == 0) continue;
+    const int st = launch_states(p[i], waves[i], smem[i], s);
+    if (st) return st;
+  }
   return CS_OK;
 }
 
