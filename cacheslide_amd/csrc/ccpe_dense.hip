@@ -499,10 +499,10 @@ int compute_units() {
 template <typename T, int D>
 int launch_dense(dense_params p, hipStream_t s) {
   // 4 waves per workgroup (128 columns share a staged tile) once that gives
-  // every CU two workgroups, else 2 waves: a short call's longest walks are
-  // then spread over twice as many workgroups.
+  // three workgroups per two CUs, else 2 waves: a short call's longest walks
+  // are then spread over twice as many workgroups.
   const auto blocks = [&](int w) { return ceil_div(p.nq, kCols * w / p.group) * p.hkv; };
-  const int waves = blocks(4) < 2 * compute_units() ? 2 : 4;
+  const int waves = blocks(4) < 3 * compute_units() / 2 ? 2 : 4;
   p.rows_per_wg = kCols * waves / p.group;
   const int64_t total = blocks(waves);
   CS_REQUIRE(total < (1ll << 31), "grid too large");

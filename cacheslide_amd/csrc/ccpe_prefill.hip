@@ -1094,10 +1094,13 @@ int prepare_prefill(const void* q, int64_t q_s_batch, int64_t q_s_tok, int64_t q
   const int tab_stride = (max_positions + 1) | 1;
   auto tab_bytes = [&](int w) { return sizeof(float) * kCols * w * static_cast<size_t>(tab_stride); };
   int waves = 2 * (tab_bytes(4) + kStaticLds) <= kLdsLimit ? 4 : (tab_bytes(8) + kStaticLds <= kLdsLimit ? 8 : 4);
-  // A launch of fewer 4-wave workgroups than two per CU (a selective call's
-  // few hundred rows) runs 2-wave workgroups: twice as many workgroups share
-  // the longest key walks.
-  if (static_cast<int64_t>(batch) * hkv * ceil_div(nq, kCols * 4 / group) < 2 * device_cus() &&
+  // A launch of fewer 4-wave workgroups than three per two CUs (a selective
+  // call's few hundred rows) runs 2-wave workgroups: twice as many workgroups
+  // share the longest key walks.  With more, the half-used tiles cost more
+  // than the balance gives: 5 requests of 333 rows (440 workgroups) 198 us
+  // against 138, 2000 rows of one (504) 129 against 109; 1000 rows (256) 74
+  // against 78.
+  if (static_cast<int64_t>(batch) * hkv * ceil_div(nq, kCols * 4 / group) < 3 * device_cus() / 2 &&
       2 * (tab_bytes(2) + kStaticLds) <= kLdsLimit)
     waves = 2;
   // a caller with few rows per workgroup (one per request) asks for narrow ones
