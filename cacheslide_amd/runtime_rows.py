@@ -61,9 +61,14 @@ class LayerRows:
     residual: Tensor | None
     restored: Tensor  # int64 [1], rows restored from the snapshot
     flags: Tensor  # int32 [1]
+    block: Tensor | None = None  # int64 [2] holding both: restored, then flags
 
     def check(self) -> int:
         """One readback: raise the recorded failure, else return the restored count."""
+        if self.block is not None:
+            count, bits = self.block.tolist()
+            _raise_row_flags(bits & 0xFFFFFFFF)
+            return count
         bits = read_flags(self.flags)[0]
         _raise_row_flags(bits)
         return int(self.restored.item())
@@ -112,12 +117,13 @@ def next_layer_rows(
             raise ValueError(f"{name} dtype differs from hidden")
     out_h = hidden.new_empty((len(active), hidden.shape[1]))
     out_r = None if residual is None else torch.empty_like(out_h)
-    restored = torch.zeros(1, dtype=torch.long, device=device)
-    flags = new_flags(device)
+    # the count and the flags in one block: one fill, one readback
+    block = torch.zeros(2, dtype=torch.long, device=device)
+    restored, flags = block[:1], block[1:].view(torch.int32)[:1]
     call("cs_rows_remap", vref(hidden), vref(residual), vref(snap_h), vref(snap_r), vref(out_h), vref(out_r),
          ptr(previous), len(previous), ptr(active), len(active), ptr(fixed), len(fixed), ptr(restored),
          ptr(flags), stream)
-    rows = LayerRows(out_h, out_r, restored, flags)
+    rows = LayerRows(out_h, out_r, restored, flags, block)
     if check:
         rows.check()
     return rows
