@@ -1005,8 +1005,10 @@ struct split_plan {
 // workgroups takes the time of its longest split.  Split 0 keeps at least 4 P
 // keys (and 256): with gates around 1/2 its mass is then twice the P-1 that
 // lets the other splits stand, where a shorter one would leave the next
-// splits to the finish launch, one after another.  The finer plan must fit
-// the workspace (bytes < 0: no limit).
+// splits to the finish launch, one after another.  One request of 1500 keys,
+// 32 heads over 8: 41 us a call with 1024-key splits, 21 with 128; a decoder
+// layer's attention of 8 requests of 1900 keys 50 and 25.  The finer plan must
+// fit the workspace (bytes < 0: no limit).
 split_plan plan_splits(int64_t batch, int64_t hq, int64_t hkv, int64_t max_nk, int32_t split, int32_t npos,
                        int64_t bytes) {
   split_plan best{split, split, ceil_div(max_nk, split)};

@@ -35,7 +35,10 @@ from .ccpe import (SharedRuns, ccpe_decode_paged, ccpe_decode_shared, decode_sha
 from .position import CoPE
 
 HEAD_DIM = 128
-FUSED_BATCH = 32   # requests up to which a step's projections are cs_decoder_* launches
+# Requests up to which a step's projections are cs_decoder_* launches: 16 heads
+# over 4, FFN 5632, 4 layers, 1000 keys a request, per step 305 us (library
+# calls 773) at 1 request, 493 (761) at 32, the most those kernels take.
+FUSED_BATCH = 32
 
 
 @dataclass(frozen=True)
