@@ -178,12 +178,15 @@ class PagedDecoder:
         s = self.shape
 
         def plain(t, dtype, *dims):
-            return t.dtype == dtype and t.shape == dims and t.is_contiguous() and t.device == caches[0].device
+            return (t.dtype == dtype and t.shape == dims and t.is_contiguous() and t.device == caches[0].device
+                    and t.data_ptr() % 16 == 0)
 
         wide = (s.heads + 2 * s.kv_heads) * HEAD_DIM
         bf16, b = torch.bfloat16, ids.shape[0]
         return (
-            s.ffn % 32 == 0 and len(caches) == len(self.layers) and plain(positions, torch.long, b)
+            s.ffn % 32 == 0 and len(caches) == len(self.layers)
+            and positions.dtype == torch.long and positions.shape == (b,) and positions.is_contiguous()
+            and positions.device == caches[0].device
             and ids.dtype == torch.long and ids.ndim == 1
             and block_table.dtype == torch.int32 and block_table.ndim == 2 and block_table.stride(1) == 1
             and block_table.shape[0] == b and block_table.shape[1] > 0 and block_table.device == caches[0].device
