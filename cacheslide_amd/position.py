@@ -621,9 +621,6 @@ def cope_attention(
         # decides between the result and the reference's error
         ck.flags[:1].bitwise_and_(~_hip.FLAG_POLICY_GENERIC)
 
-    policy = canonical is not None or selected is not None
-    if default_keys and not policy:
-        key_positions = torch.arange(nk, device=device)
     if fixed_positions is not None:
         call("cs_check_bias_positions", vref(fixed_positions), cope.max_positions, ck.flags_ptr, ck.stream)
 
@@ -642,7 +639,7 @@ def cope_attention(
     chunk_flags = None
     lowered = None
     sel_rows = fixed_keys = None
-    if policy:
+    if canonical is not None or selected is not None:
         lowered, sel_rows, fixed_keys = lower_policies(canonical, selected, device, query_positions, key_positions, nk)
     if canonical is not None:
         if lowered.reason or not lowered.fits(hq):
@@ -676,7 +673,7 @@ def cope_attention(
     # for the device per call).
     flags_value = None
     chunk_values = None
-    if (policy and default_keys
+    if ((selected is not None or canonical is not None) and default_keys
             and _policy_fast_ok(query, key, value, e, cope, amask, visibility_mask, fixed_positions,
                                 return_positions, lowered if canonical is not None else None)
             and _policy_prefill(args, query, key, ck)):

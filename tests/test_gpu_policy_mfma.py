@@ -22,6 +22,8 @@ longer), optionally perturbed or missing some ordinals.
 
 from __future__ import annotations
 
+import dataclasses
+
 import numpy as np
 import pytest
 import torch
@@ -430,3 +432,18 @@ def test_key_split_selected_call_matches_generic_and_oracle(device, monkeypatch,
     want = orc.cope_attention(q[rows[pick]], k, v, e, rows[pick], visibility_transform=oracle_visibility,
                               query_chunk_size=64)
     assert_close_bf16(actual[1][torch.from_numpy(pick).to(device)], want)
+
+
+def test_mismatched_profile_is_ignored_without_fixed_rows(device, monkeypatch):
+    """A profile of another checkpoint is an error only when a query row is
+    fixed: over recomputed rows the generic kernel takes the call without it."""
+    q, k, v, e, _, plan, cal, ordinals, _ = scenario(31, a=60, dyn=20, b=40, n_sel=10)
+    rows = np.arange(60, 80)
+    profile = dataclasses.replace(profile_for(plan, cal, ordinals), checkpoint_id="another")
+    expected = orc.cope_attention(q[rows], k, v, e, rows)
+    actual, called = device_run(q, k, v, e, rows, plan, profile, "strict_contextual", None, 64, device, monkeypatch)
+    compare(("ok", expected), actual)
+    assert "cs_ccpe_attention" in called
+    actual, _ = device_run(q, k, v, e, np.arange(59, 80), plan, profile, "strict_contextual", None, 64, device,
+                           monkeypatch)
+    assert actual[:2] == ("error", ValueError)
