@@ -452,8 +452,10 @@ extern "C" int cs_page_copy(const cs_view* cache, const int64_t* src_blocks,
   hipStream_t s = as_stream(stream);
   const int64_t run = c.heads * c.bs * c.rec_bytes;
   const int64_t segs = ceil_div(run, kRunBytes);
+  // A launch holds fewer than 2^32 work-items: 2^24 workgroups and more (64 GB
+  // in 4 KB pages) go to the grid-stride kernel below.
   if (w == 16 && c.s_off == c.rec_bytes && c.s_head == c.bs * c.rec_bytes && c.layers > 0 && segs > 0 &&
-      n * c.layers * segs < (1ll << 31)) {
+      n * c.layers * segs < (1ll << 24)) {
     hipLaunchKernelGGL(page_run_copy_kernel, dim3(static_cast<uint32_t>(n * c.layers * segs)), dim3(256), 0, s, c,
                        src_blocks, dst_blocks, run, static_cast<uint32_t>(segs));
     CS_LAUNCH_CHECK("page_copy");

@@ -141,6 +141,20 @@ def test_page_copy_of_compact_pages(device, shape):
     assert torch.equal(cache, want)
 
 
+@pytest.mark.parametrize("n", [2**24 - 1, 2**24])
+def test_page_copy_of_the_most_workgroups(device, n):
+    """A workgroup per 4 KB page up to the work-items one launch holds, the
+    grid-stride kernel from there on: pages at both ends of a list whose other
+    entries name no block."""
+    cache = torch.randn((128, 1, 16, 128), generator=torch.Generator().manual_seed(6)).to(torch.bfloat16).to(device)
+    want = torch.cat([cache[64:], cache[64:]])
+    src, dst = (torch.full((n,), -1, device=device) for _ in range(2))
+    dst[:32], dst[-32:] = torch.arange(32, device=device), torch.arange(32, 64, device=device)
+    src[:32], src[-32:] = dst[:32] + 64, dst[-32:] + 64
+    relocate.copy_pages(cache, src, dst, check=False)
+    assert torch.equal(cache, want)
+
+
 # ------------------------------------------------------------ reference fixtures
 def fixture_arena(device, max_selected=2):
     # tests/test_paged.py:13-23 (non-contiguous cache: every second element)
