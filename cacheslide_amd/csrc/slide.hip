@@ -452,9 +452,12 @@ extern "C" int cs_page_copy(const cs_view* cache, const int64_t* src_blocks,
   hipStream_t s = as_stream(stream);
   const int64_t run = c.heads * c.bs * c.rec_bytes;
   const int64_t segs = ceil_div(run, kRunBytes);
-  // A launch holds fewer than 2^32 work-items: 2^24 workgroups and more (64 GB
-  // in 4 KB pages) go to the grid-stride kernel below.
-  if (w == 16 && c.s_off == c.rec_bytes && c.s_head == c.bs * c.rec_bytes && c.layers > 0 && segs > 0 &&
+  // A run of fewer bytes than a workgroup loads at once leaves threads idle:
+  // 2^20 pages of 16 bytes took 737 us (31 by the kernel below), of 1 KB 784
+  // (481), 2^19 of 2 KB 489 (476), 2^18 of 4 KB 430 (469).  And a launch holds
+  // fewer than 2^32 work-items: 2^24 workgroups and more (64 GB in 4 KB pages)
+  // go to that kernel too.
+  if (w == 16 && c.s_off == c.rec_bytes && c.s_head == c.bs * c.rec_bytes && c.layers > 0 && run >= kRunBytes / kRunVec &&
       n * c.layers * segs < (1ll << 24)) {
     hipLaunchKernelGGL(page_run_copy_kernel, dim3(static_cast<uint32_t>(n * c.layers * segs)), dim3(256), 0, s, c,
                        src_blocks, dst_blocks, run, static_cast<uint32_t>(segs));

@@ -128,7 +128,7 @@ def test_free_list_bits_left_after_acquire(device, nbits, count):
     np.testing.assert_array_equal(fl.free_mask().numpy(), left)
 
 
-@pytest.mark.parametrize("shape", [(2, 9, 3, 4, 8), (3, 9, 8, 16, 256), (7, 2, 16, 96)])
+@pytest.mark.parametrize("shape", [(2, 9, 3, 4, 8), (3, 9, 8, 16, 256), (7, 2, 16, 96), (9, 1, 16, 128), (9, 1, 17, 120)])
 def test_page_copy_of_compact_pages(device, shape):
     """Pages that are one run of bytes, of less than, exactly and more than the
     bytes a workgroup copies, and ones past the cache's blocks (skipped)."""
