@@ -7,13 +7,13 @@
 // keys before split r-1 (plan_splits).  Split 0 is computed exactly (carry 0).
 // Every other split assumes that the gate mass of the keys to its right is
 // already >= P-1, which makes every position in it P-1 and the bias the row
-// constant QE[P-1]; it records its own gate total.  A second launch, one
-// workgroup per (request, KV head), forms the splits' true carries (sum of the
-// totals to their right) from the right-most split until every head's carry
-// reaches P-1 -- carries only grow, so the splits that need it are a prefix --
-// recomputes those splits exactly, and merges the per-split (max, sum,
-// accumulator) triples into the output rows.  Split 0's workgroups lead the
-// first launch's grid.
+// constant QE[P-1]; it records its own gate total.  A second launch forms the
+// splits' true carries (sum of the totals to their right) of each (request, KV
+// head) from the right-most split until every head's carry reaches P-1 --
+// carries only grow, so the splits that need it are a prefix -- recomputes
+// those splits exactly, and merges the per-split (max, sum, accumulator)
+// triples into the output rows (decode_finish_kernel).  Split 0's workgroups
+// lead the first launch's grid.
 //
 // Inside a split each of the 4 wavefronts owns a contiguous quarter of the
 // keys and walks it in tiles of 16 keys from the right.  Per tile:
@@ -84,8 +84,10 @@ struct decode_params {
   const float* e;
   int32_t npos;
   int32_t split0, split, smax;  // keys of split 0 and of the others, splits at most
+  int32_t fix_wgs;     // finish workgroups per (request, KV head): 1, or smax
   double* tot;         // [B, hq, smax] gate totals
-  double* carry;       // [B, hq, smax] gate mass to the right of each split
+  double* carry;       // [B, hq, smax] gate mass to the right of each split (split 0's entry
+                       // of a group's first head: the group's fix_count)
   float* mx;           // [B, hq, smax] running max (log2 domain)
   float* sm;           // [B, hq, smax] sum of exp2
   float* acc;          // [B, hq, smax, 128]
@@ -133,6 +135,7 @@ struct smem_t {
   float wave_l[kWaves][G];
   float red[2][2];
   int fix_end;  // group finish: splits 1 .. fix_end-1 are recomputed
+  uint32_t fix_done;  // splits of the group recomputed, this workgroup's included
 };
 
 struct split_ctx {
@@ -724,14 +727,15 @@ __device__ void run_exact(const decode_params& p, smem_t<G>& s, const split_ctx&
 // ---- finish of one (request, KV head) group ---------------------------------
 
 // Carries of splits 1, 2, ... (sum of the split totals to their right, fp64,
-// accumulated from the right-most split) into p.carry, 64 splits at a time
-// (wave 0, lane i: the total of split base+i, the carry of split base+i+1),
-// up to the first split at which every head's carry has reached P-1;
-// s.fix_end is that split (or `splits`).  Gate totals are sums of sigmoids, so
-// carries never decrease along the splits and no later split needs
-// recomputing.
+// accumulated from the right-most split), 64 splits at a time (wave 0, lane i:
+// the total of split base+i, the carry of split base+i+1), up to the first
+// split at which every head's carry has reached P-1; s.fix_end is that split
+// (or `splits`).  Gate totals are sums of sigmoids, so carries never decrease
+// along the splits and no later split needs recomputing.  A group of one
+// finish workgroup (own < 0) leaves the carries in p.carry; one of several
+// keeps the carry of its own split in s.carry.
 template <int G>
-__device__ void plan_group(const decode_params& p, smem_t<G>& s, int b, int h0, int splits) {
+__device__ void plan_group(const decode_params& p, smem_t<G>& s, int b, int h0, int splits, int own) {
   if (threadIdx.x >= 64) return;
   const int lane = threadIdx.x;
   const double top = static_cast<double>(p.npos - 1);
@@ -756,7 +760,10 @@ __device__ void plan_group(const decode_params& p, smem_t<G>& s, int b, int h0, 
       }
       const double carry = carry_in[h] + x;
       if (has_next) {
-        p.carry[ws_index(p, b, h0 + h, r + 1)] = carry;
+        if (own < 0)
+          p.carry[ws_index(p, b, h0 + h, r + 1)] = carry;
+        else if (own == r + 1)
+          s.carry[h] = carry;
         below |= carry < top;  // false for NaN
       }
       carry_in[h] += __shfl(x, 63, 64);
@@ -783,6 +790,34 @@ __device__ void fixup_group(const decode_params& p, smem_t<G>& s, int b, int kvh
     run_exact<G, PAGED>(p, s, c, false, bad);
     __syncthreads();
   }
+}
+
+// Splits of a group recomputed so far, by its finish workgroups.
+__device__ inline uint32_t* fix_count(const decode_params& p, int b, int h0) {
+  return reinterpret_cast<uint32_t*>(p.carry + ws_index(p, b, h0, 0));
+}
+
+// Exact recomputation of split `own` (carry in s.carry) by one of its group's
+// finish workgroups.  True, in every thread, for the last of the group's
+// s.fix_end - 1 such workgroups, which then sees the partials of all.
+template <int G, bool PAGED>
+__device__ bool fixup_one(const decode_params& p, smem_t<G>& s, int b, int kvh, int own, bool& bad) {
+  split_ctx c;
+  make_ctx(p, b, kvh, own, c);
+  run_exact<G, PAGED>(p, s, c, false, bad);
+  // Every wave's stores have reached this XCD's L2, which one wave then writes
+  // back before the count (a write-back per wave made 128 such workgroups 5 us
+  // slower); the last workgroup drops what it holds of the others' lines.
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
+    s.fix_done = atomicAdd(fix_count(p, b, c.h0), 1u) + 1;
+  }
+  __syncthreads();
+  const bool last = static_cast<int>(__builtin_amdgcn_readfirstlane(s.fix_done)) == s.fix_end - 1;
+  if (last) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+  return last;
 }
 
 // Merge of the split partials of two query heads, threads 0..127 for head ha
@@ -864,12 +899,12 @@ __device__ void combine_pair(const decode_params& p, smem_t<G>& s, int b, int ha
 // holds split r's max and sum, whose weight reaches every lane through
 // v_readlane.  Returns false, with the plan in s.fix_end and nothing
 // written, when some split must be recomputed first; the value is the same
-// in every thread.
+// in every thread.  own > 0: that has been done, the partials are merged.
 template <int G>
 constexpr int fast_chunks() { return (G + 1) / 2 > 2 ? 2 : 4; }
 
 template <int G, int NCH>
-__device__ bool merge_fast(const decode_params& p, smem_t<G>& s, int b, int h0, int splits) {
+__device__ bool merge_fast(const decode_params& p, smem_t<G>& s, int b, int h0, int splits, int own) {
   constexpr int NH = (G + 1) / 2;
   constexpr int R = 16 * NCH;
   static_assert(R <= 64 && NH * R <= 128, "partials held per thread");
@@ -888,9 +923,11 @@ __device__ bool merge_fast(const decode_params& p, smem_t<G>& s, int b, int h0, 
     mv[j] = p.mx[w0 + rl];
     lv[j] = p.sm[w0 + rl];
   }
-  plan_group<G>(p, s, b, h0, splits);
-  __syncthreads();
-  if (__builtin_amdgcn_readfirstlane(s.fix_end) > 1) return false;
+  if (own <= 0) {
+    plan_group<G>(p, s, b, h0, splits, own);
+    __syncthreads();
+    if (__builtin_amdgcn_readfirstlane(s.fix_end) > 1) return false;
+  }
 #pragma unroll
   for (int j = 0; j < NH; ++j) {
     const int h = half + 2 * j;
@@ -909,17 +946,19 @@ __device__ bool merge_fast(const decode_params& p, smem_t<G>& s, int b, int h0, 
 }
 
 template <int G>
-__device__ bool merge_fast_any(const decode_params& p, smem_t<G>& s, int b, int h0, int splits) {
+__device__ bool merge_fast_any(const decode_params& p, smem_t<G>& s, int b, int h0, int splits, int own) {
   switch ((splits + 15) >> 4) {
-    case 1: return merge_fast<G, 1>(p, s, b, h0, splits);
-    case 2: return merge_fast<G, 2>(p, s, b, h0, splits);
-    case 3: if constexpr (fast_chunks<G>() >= 3) return merge_fast<G, 3>(p, s, b, h0, splits); break;
-    case 4: if constexpr (fast_chunks<G>() >= 4) return merge_fast<G, 4>(p, s, b, h0, splits); break;
+    case 1: return merge_fast<G, 1>(p, s, b, h0, splits, own);
+    case 2: return merge_fast<G, 2>(p, s, b, h0, splits, own);
+    case 3: if constexpr (fast_chunks<G>() >= 3) return merge_fast<G, 3>(p, s, b, h0, splits, own); break;
+    case 4: if constexpr (fast_chunks<G>() >= 4) return merge_fast<G, 4>(p, s, b, h0, splits, own); break;
     default: break;
   }
   // no key, or more splits than the registers hold: plan only
-  plan_group<G>(p, s, b, h0, splits);
-  __syncthreads();
+  if (own <= 0) {
+    plan_group<G>(p, s, b, h0, splits, own);
+    __syncthreads();
+  }
   return false;
 }
 
@@ -942,6 +981,7 @@ __global__ void __launch_bounds__(kThreads) decode_main_kernel(decode_params p) 
   if (!make_ctx(p, b, kvh, r, c)) return;
   bool bad = false;
   if (r == 0) {
+    if (threadIdx.x == 0 && p.fix_wgs > 1) *fix_count(p, b, c.h0) = 0;
     if (threadIdx.x < G) s.carry[threadIdx.x] = 0.0;
     run_exact<G, PAGED>(p, s, c, true, bad);
   } else {
@@ -950,18 +990,39 @@ __global__ void __launch_bounds__(kThreads) decode_main_kernel(decode_params p) 
   if (bad) atomicOr(p.flags, CS_FLAG_BLOCK_INVALID);
 }
 
-// One workgroup per (request, KV head): carries, recomputation of the splits
-// whose carry is below P-1, and the merge into the output rows.
+// Per (request, KV head): carries, recomputation of the splits whose carry is
+// below P-1, and the merge into the output rows.  One workgroup, which
+// recomputes such splits one after another, or in a call of finer splits
+// (plan_splits) one per split: workgroup r > 0 recomputes split r when it has
+// to be, and the last to end merges; workgroup 0 merges when none has to be.
+// One after another, short splits of low gates cost such a call more than
+// coarse ones (a call of 1500 keys, 32 heads over 8, P = 64, gates around 0.1 /
+// 0.05 / 0.03: 66 / 116 / 125 us, with 1024-key splits 41 / 78 / 78); side by
+// side it takes 33 / 34 / 34, and 8 requests of 1900 keys, 16 heads over 4, at
+// most 40 (160; 80 with 1024-key splits).
 template <int G, bool PAGED>
 __global__ void __launch_bounds__(kThreads) decode_finish_kernel(decode_params p) {
   __shared__ smem_t<G> s;
   if (p.gate != nullptr && __builtin_amdgcn_readfirstlane(*p.gate) == 0) return;  // before any barrier
+  const int own = static_cast<int>(blockIdx.y);
   const int b = blockIdx.x / p.hkv, kvh = blockIdx.x % p.hkv;
   const int h0 = kvh * G;
   const int splits = splits_of(p, keys_of(p, b));  // no key: zero rows (the call is flagged)
   bool bad = false;
-  if (merge_fast_any<G>(p, s, b, h0, splits)) return;
-  fixup_group<G, PAGED>(p, s, b, kvh, bad);
+  if (own > 0) {
+    if (own >= splits) return;
+    plan_group<G>(p, s, b, h0, splits, own);
+    __syncthreads();
+    if (own >= __builtin_amdgcn_readfirstlane(s.fix_end)) return;
+    const bool last = fixup_one<G, PAGED>(p, s, b, kvh, own, bad);
+    if (bad) atomicOr(p.flags, CS_FLAG_BLOCK_INVALID);
+    if (!last) return;
+  }
+  if (merge_fast_any<G>(p, s, b, h0, splits, p.fix_wgs > 1 ? own : -1)) return;
+  if (p.fix_wgs == 1)
+    fixup_group<G, PAGED>(p, s, b, kvh, bad);
+  else if (own == 0 && __builtin_amdgcn_readfirstlane(s.fix_end) > 1)
+    return;  // the last of the recomputing workgroups merges
   for (int h = 0; h < G; h += 2) combine_pair<G>(p, s, b, h0 + h, h + 1 < G ? h0 + h + 1 : -1, splits);
   if (bad) atomicOr(p.flags, CS_FLAG_BLOCK_INVALID);
 }
@@ -971,7 +1032,7 @@ void launch_split_kernels(const decode_params& p, hipStream_t s) {
   const int64_t main_grid = static_cast<int64_t>(p.smax) * p.hkv * p.batch;
   hipLaunchKernelGGL((decode_main_kernel<G, PAGED>), dim3(static_cast<uint32_t>(main_grid)),
                      dim3(kThreads), 0, s, p);
-  hipLaunchKernelGGL((decode_finish_kernel<G, PAGED>), dim3(static_cast<uint32_t>(p.hkv * p.batch)),
+  hipLaunchKernelGGL((decode_finish_kernel<G, PAGED>), dim3(static_cast<uint32_t>(p.hkv * p.batch), p.fix_wgs),
                      dim3(kThreads), 0, s, p);
 }
 
@@ -1000,15 +1061,15 @@ struct split_plan {
 
 // The splits of a call: `split` keys each while that gives the chip enough
 // workgroups, else `split` halved until it does (128 keys at the least, 32
-// splits at the most: those are merged in one round of loads).  A workgroup
-// draws about 10 bytes a cycle whatever its shape, so a call of few
+// splits at the most: groups of every size merge those in one round of loads).
+// A workgroup draws about 10 bytes a cycle whatever its shape, so a call of few
 // workgroups takes the time of its longest split.  Split 0 keeps at least 4 P
 // keys (and 256): with gates around 1/2 its mass is then twice the P-1 that
-// lets the other splits stand, where a shorter one would leave the next
-// splits to the finish launch, one after another.  One request of 1500 keys,
-// 32 heads over 8: 41 us a call with 1024-key splits, 21 with 128; a decoder
-// layer's attention of 8 requests of 1900 keys 50 and 25.  The finer plan must
-// fit the workspace (bytes < 0: no limit).
+// lets the other splits stand, where a shorter one would have the finish launch
+// recompute the next ones.  One request of 1500 keys, 32 heads over 8: 41 us a
+// call with 1024-key splits, 21 with 128; a decoder layer's attention of 8
+// requests of 1900 keys 50 and 25.  The finer plan must fit the workspace
+// (bytes < 0: no limit).
 split_plan plan_splits(int64_t batch, int64_t hq, int64_t hkv, int64_t max_nk, int32_t split, int32_t npos,
                        int64_t bytes) {
   split_plan best{split, split, ceil_div(max_nk, split)};
@@ -1142,9 +1203,11 @@ int prepare_decode(const void* q, int64_t q_s_batch, int64_t q_s_head, int32_t b
 // cs_ccpe_decode_workspace_bytes), carve it and launch the kernels.
 int launch_decode(decode_params& p, void* workspace, int64_t bytes, void* stream) {
   const split_plan f = plan_splits(p.batch, p.hq, p.hkv, p.max_nk, p.split, p.npos, bytes);
+  const bool finer = f.split < p.split;
   p.split0 = f.split0;
   p.split = f.split;
   p.smax = static_cast<int32_t>(f.smax);
+  p.fix_wgs = finer ? p.smax : 1;
   const int64_t n = static_cast<int64_t>(p.batch) * p.hq * p.smax;
   char* ws = static_cast<char*>(workspace);
   p.tot = reinterpret_cast<double*>(ws);

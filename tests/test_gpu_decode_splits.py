@@ -18,15 +18,15 @@ from tests.test_gpu_ccpe import cope_on
 pytestmark = pytest.mark.gpu
 
 
-def setup(device, lens, hq, hkv, npos, low_gates=False):
+def setup(device, lens, hq, hkv, npos, low_gates=0.0):
     blocks, table, rows = paged_layout(lens, hkv, 16, 128, seed=sum(lens))
     cache = torch.zeros((blocks, hkv, 16, 256), dtype=torch.bfloat16)
     keys = [seeded((n, hkv, 128), 7 + i, dtype=torch.bfloat16) for i, n in enumerate(lens)]
     vals = [seeded((n, hkv, 128), 17 + i, dtype=torch.bfloat16) for i, n in enumerate(lens)]
     q = seeded((len(lens), hq, 128), 3, dtype=torch.bfloat16)
-    if low_gates:                       # q.k / sqrt(128) around -5: gates of 0.007
+    if low_gates:                       # q.k / sqrt(128) around -7.2 low_gates: gates of 0.007 at 0.7
         q = q.abs()
-        keys = [-(k.abs() * 0.7) for k in keys]
+        keys = [-(k.abs() * low_gates) for k in keys]
     fill_paged(cache, rows, keys, vals)
     e = seeded((128, npos), 5, scale=0.1)
     want = np.concatenate([orc.cope_attention(acc_np(q[i:i + 1]), acc_np(k), acc_np(v), e.numpy(),
@@ -46,7 +46,7 @@ def test_small_calls_match_the_oracle(device, lens, npos):
 
 @pytest.mark.parametrize("lens", [[700], [1500, 129]])
 def test_small_calls_with_low_gates(device, lens):
-    args, want = setup(device, lens, 8, 1, 64, low_gates=True)
+    args, want = setup(device, lens, 8, 1, 64, low_gates=0.7)
     assert_close_bf16(ccpe_decode_paged(*args, max_context=max(lens)), want)
 
 
@@ -61,3 +61,19 @@ def test_a_workspace_for_the_plain_split_is_taken(device):
     out = ccpe_decode_paged(*args, max_context=1500, workspace=both[:small.numel()], flags=flags)
     assert_close_bf16(out, want)
     assert bool((both[small.numel():] == 77).all())
+
+
+@pytest.mark.parametrize("hq,hkv,npos", [(8, 1, 64), (32, 8, 64), (6, 2, 128), (3, 3, 16)])
+@pytest.mark.parametrize("lens", [[257], [1500], [900, 1500, 333], [4200]])
+@pytest.mark.parametrize("low_gates", [0.2, 0.35, 0.7])
+def test_splits_recomputed_side_by_side(device, lens, hq, hkv, npos, low_gates):
+    """Gates of 0.2 to 0.007: some or all of the later splits are recomputed,
+    each by a workgroup of its own, and the last to end merges: in the same
+    order whichever that is."""
+    args, want = setup(device, lens, hq, hkv, npos, low_gates=low_gates)
+    workspace = decode_workspace(len(lens), hq, max(lens), 1024, device)
+    first = ccpe_decode_paged(*args, max_context=max(lens), workspace=workspace)
+    assert_close_bf16(first, want)
+    for _ in range(20):
+        workspace.fill_(0xFF)
+        assert torch.equal(ccpe_decode_paged(*args, max_context=max(lens), workspace=workspace), first)
