@@ -258,7 +258,7 @@ ccpe_dense_kernel(dense_params p) {
   }
 
   const int64_t wgmax = wg_max_pos;  // written before the barriers above
-  const int kend = static_cast<int>(wgmax + 1 < p.nk ? wgmax + 1 : p.nk);  // keys [0, kend)
+  const int kend = wgmax < p.nk ? static_cast<int>(wgmax) + 1 : p.nk;  // keys [0, kend); any int64 position
   const int ntiles = (kend + kTileN - 1) / kTileN;
   const int qp32 = qp < 0 ? -1 : static_cast<int>(qp < p.nk ? qp : p.nk);
   const int wmax32 = __builtin_amdgcn_readfirstlane(wmax < 0 ? -1 : static_cast<int>(wmax < p.nk ? wmax : p.nk));

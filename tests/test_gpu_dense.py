@@ -37,15 +37,16 @@ def cope_of(device, table):
     return cope
 
 
-def check(device, dtype, d, hq, hkv, n, rows, npos, strided=False, seed=0):
+def check(device, dtype, d, hq, hkv, n, rows, npos, strided=False, seed=0, positions=None):
     width = d + (16 // torch.empty((), dtype=dtype).element_size() if strided else 0)
     q, k, v = (seeded((n, heads, width), seed + i, dtype=dtype) for i, heads in enumerate((hq, hkv, hkv)))
     e = seeded((d, npos), seed + 3, scale=0.1)
     cope = cope_of(device, e)
     qd, kd, vd = (x.to(device)[..., :d] for x in (q[rows], k, v))
-    out = cope_attention(qd, kd, vd, cope, torch.from_numpy(rows).to(device)).cpu().double().numpy()
+    positions = rows if positions is None else positions
+    out = cope_attention(qd, kd, vd, cope, torch.from_numpy(positions).to(device)).cpu().double().numpy()
     wide = [x.double().numpy()[..., :d] for x in (q[rows], k, v)]
-    expected = orc.cope_attention(*wide, e.double().numpy(), rows)
+    expected = orc.cope_attention(*wide, e.double().numpy(), positions)
     diff = out - expected
     assert np.linalg.norm(diff) <= REL[dtype] * np.linalg.norm(expected)
     assert np.abs(diff).max() <= REL[dtype] * np.abs(expected).max()
@@ -95,3 +96,13 @@ def test_dense_values_past_the_range_take_the_generic_kernel(device, called):
     expected = orc.cope_attention(*(x.cpu().double().numpy() for x in (q, k, large)), np.zeros((64, 8)), np.arange(40))
     assert np.abs(out.cpu().double().numpy() - expected).max() <= 1e-5 * np.abs(expected).max()
     assert called.count("cs_ccpe_attention") == 3
+
+
+@pytest.mark.parametrize("dtype,d", [(torch.float16, 128), (torch.float32, 64)])
+def test_dense_largest_query_position(device, called, dtype, d):
+    """A row past every key, up to the largest int64, sees all of them."""
+    rows = np.arange(40, 70)
+    positions = rows.copy()
+    positions[[3, 29]] = 2**63 - 1, 2**31 + 5
+    check(device, dtype, d, 4, 2, 70, rows, 64, seed=2, positions=positions)
+    assert "cs_ccpe_attention" not in called
