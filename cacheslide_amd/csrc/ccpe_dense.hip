@@ -12,8 +12,8 @@
 //
 // What bounds it.  f32: the matrix cores (v_mfma_f32_32x32x2_f32, 64 of 64
 // cycles for each of the two products of a 32 x 32 tile at D = 128).  16-bit
-// types: the position and softmax arithmetic of the VALU beside 8 + 16 MFMAs
-// of 32 cycles.  Both are contractions, so a wave that computes one (row,
+// types: the position and softmax arithmetic of the VALU beside the MFMAs of 32
+// cycles (f16 at D = 128: 8 of Q.K and 40 of P.V a tile).  Both are contractions, so a wave that computes one (row,
 // head) pair on scalar dot products -- the generic kernel -- is two orders of
 // magnitude away: at 1000 tokens, 32 query heads over 8 KV heads, D = 128,
 // f16, that kernel took 4150 us and this one takes 88; f32 at 2048 tokens, 16
@@ -28,13 +28,20 @@
 // computed, two workgroups per CU cover each other's barriers.  Rows are
 // padded so that the 16-byte K reads of 16 lanes fall in distinct banks.
 //
-// Precision is that of the generic kernel: products of the inputs are summed
-// in fp32, gates are summed in fp64, and a probability keeps its fp32 value:
-// f32 multiplies it in fp32, f16 as two f16 terms (22 bits), bf16 as three
-// bf16 terms (24 bits).  The table QE uses fp32 products (f32) or Q and E
-// split into bf16 terms that keep 24 bits of their product.  2-norm error
-// against fp64 over 40 .. 2048 tokens: f32 1.04e-6 (generic kernel 1.09e-6,
-// lower here at every size), 16-bit types that of their output's rounding.
+// Precision.  Products of the inputs are summed in fp32 and gates in fp64, as
+// in the generic kernel, and a probability keeps its fp32 value whatever its
+// size: f32 multiplies it in fp32, the 16-bit types as three bf16 terms (24
+// bits, the range of fp32) by V in bf16, an f16 V as two bf16 terms, which hold
+// it exactly.  (As two f16 terms a probability ends at 2^-25: 40000 keys below
+// it, 8e-4 of the softmax, left the output but not its norm.  The bf16 terms
+// take 142 us a call at 1000 tokens, 32 heads over 8, D = 128, those 137.)
+// f32 forms gates and exponentials as the generic kernel does; the 16-bit
+// types take v_exp_f32 and v_rcp_f32, within a unit in the last place each, of
+// a score scaled once, where the generic kernel rounds the logit.  The table QE
+// uses fp32 products (f32) or Q and E split into bf16 terms that keep 24 bits
+// of their product.  2-norm error against fp64 over 40 .. 2048 tokens: f32
+// 1.04e-6 (generic kernel 1.09e-6, lower here at every size), 16-bit types that
+// of their output's rounding (2.0e-4 f16, 1.6e-3 bf16, as the generic kernel).
 //
 // Values whose arithmetic could leave the finite range (a score, a QE entry
 // or an output beyond 1e37 in magnitude, or not finite) set
@@ -73,21 +80,20 @@ struct dense_params {
 
 template <typename T> struct dense_elem;
 template <> struct dense_elem<float> {
-  static constexpr int kSize = 4, kPad = 32;
+  static constexpr int kSize = 4, kPad = 32, kVTiles = 1;
 };
 template <> struct dense_elem<f16_t> {
   static constexpr int kSize = 2, kPad = 16;
+  static constexpr int kVTiles = 2;  // V as two bf16 terms, exactly
   using vec = f16x8;
-  static constexpr int kTerms = 2;  // of a probability
   using scalar = _Float16;
   __device__ static floatx16 mfma(vec a, vec b, floatx16 c) {
     return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0);
   }
 };
 template <> struct dense_elem<bf16_t> {
-  static constexpr int kSize = 2, kPad = 16;
+  static constexpr int kSize = 2, kPad = 16, kVTiles = 1;
   using vec = bf16x8;
-  static constexpr int kTerms = 3;
   using scalar = __bf16;
   __device__ static floatx16 mfma(vec a, vec b, floatx16 c) {
     return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
@@ -142,7 +148,7 @@ ccpe_dense_kernel(dense_params p) {
   extern __shared__ __align__(16) char smem[];
   char* ks_lds = smem;
   char* vs_lds = smem + kTileN * kRow;
-  float* tab = reinterpret_cast<float*>(smem + 2 * kTileN * kRow);  // [cols][tab_stride]
+  float* tab = reinterpret_cast<float*>(smem + (1 + E::kVTiles) * kTileN * kRow);  // [cols][tab_stride]
   __shared__ int64_t wg_max_pos;
 
   const int tid = threadIdx.x, lane = tid & 63;
@@ -218,7 +224,7 @@ ccpe_dense_kernel(dense_params p) {
           e1[i] = t[1];
           e2[i] = t[2];
         }
-        if constexpr (E::kTerms == 2) {
+        if constexpr (__is_same(T, f16_t)) {
           // an f16 value is the sum of two bf16 values
           const f16x8 qh = __builtin_bit_cast(f16x8, qb[ks]);
 #pragma unroll
@@ -285,7 +291,21 @@ ccpe_dense_kernel(dense_params p) {
       const int i = tid + kThreads * r;
       const int at = (i / kChunks) * kRow + 16 * (i % kChunks);
       *reinterpret_cast<uint4*>(ks_lds + at) = kr[r];
-      *reinterpret_cast<uint4*>(vs_lds + at) = vr[r];
+      if constexpr (__is_same(T, f16_t)) {
+        const f16x8 v = __builtin_bit_cast(f16x8, vr[r]);
+        bf16x8 v0, v1;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          __bf16 t[2];
+          split_bf16<2>(static_cast<float>(v[e]), t);
+          v0[e] = t[0];
+          v1[e] = t[1];
+        }
+        *reinterpret_cast<bf16x8*>(vs_lds + at) = v0;
+        *reinterpret_cast<bf16x8*>(vs_lds + kTileN * kRow + at) = v1;
+      } else {
+        *reinterpret_cast<uint4*>(vs_lds + at) = vr[r];
+      }
     }
   };
 
@@ -421,28 +441,27 @@ ccpe_dense_kernel(dense_params p) {
     } else {
 #pragma unroll
       for (int ks = 0; ks < 2; ++ks) {
-        typename E::vec pb[E::kTerms];
+        // a probability as three bf16 terms, all of its 24 bits at any size
+        bf16x8 pb[3];
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
-          float x = s[8 * ks + i];
+          __bf16 t[3];
+          split_bf16<3>(s[8 * ks + i], t);
 #pragma unroll
-          for (int w = 0; w < E::kTerms; ++w) {
-            const typename E::scalar y = static_cast<typename E::scalar>(x);
-            pb[w][i] = y;
-            x -= static_cast<float>(y);
+          for (int w = 0; w < 3; ++w) pb[w][i] = t[w];
+        }
+#pragma unroll
+        for (int db = 0; db < kDb; ++db)
+#pragma unroll
+          for (int u = E::kVTiles - 1; u >= 0; --u) {
+            const char* at = vrd16 + u * kTileN * kRow + 16 * ks * kRow + 64 * db;
+            const bf16x4_tr lo = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((CS_LDS bf16x4_tr*)at);
+            const bf16x4_tr hi = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((CS_LDS bf16x4_tr*)(at + 8 * kRow));
+            const auto va = __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+            // third term of P times second of V: below 2^-26 of the product
+#pragma unroll
+            for (int w = 2 - u; w >= 0; --w) o[db] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(va, pb[w], o[db], 0, 0, 0);
           }
-        }
-#pragma unroll
-        for (int db = 0; db < kDb; ++db) {
-          const bf16x4_tr lo = __builtin_amdgcn_ds_read_tr16_b64_v4bf16(
-              (CS_LDS bf16x4_tr*)(vrd16 + 16 * ks * kRow + 64 * db));
-          const bf16x4_tr hi = __builtin_amdgcn_ds_read_tr16_b64_v4bf16(
-              (CS_LDS bf16x4_tr*)(vrd16 + (16 * ks + 8) * kRow + 64 * db));
-          const auto va = __builtin_bit_cast(typename E::vec,
-                                             __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
-#pragma unroll
-          for (int w = E::kTerms - 1; w >= 0; --w) o[db] = E::mfma(va, pb[w], o[db]);
-        }
       }
     }
   };
@@ -508,7 +527,7 @@ int launch_dense(dense_params p, hipStream_t s) {
   CS_REQUIRE(total < (1ll << 31), "grid too large");
   p.row_blocks = static_cast<int32_t>(total / p.hkv);
   p.tab_stride = (p.npos + 1) | 1;  // entries 0 .. P, an odd number of words
-  const size_t smem = 2 * kTileN * (D * dense_elem<T>::kSize + dense_elem<T>::kPad) +
+  const size_t smem = (1 + dense_elem<T>::kVTiles) * kTileN * (D * dense_elem<T>::kSize + dense_elem<T>::kPad) +
                       sizeof(float) * kCols * waves * static_cast<size_t>(p.tab_stride);
   const dim3 grid(static_cast<uint32_t>(total)), block(64 * waves);
   if (waves == 2)

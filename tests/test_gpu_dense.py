@@ -106,3 +106,23 @@ def test_dense_largest_query_position(device, called, dtype, d):
     positions[[3, 29]] = 2**63 - 1, 2**31 + 5
     check(device, dtype, d, 4, 2, 70, rows, 64, seed=2, positions=positions)
     assert "cs_ccpe_attention" not in called
+
+
+@pytest.mark.parametrize("dtype,d", [(torch.float16, 128), (torch.float16, 64), (torch.bfloat16, 64)])
+@pytest.mark.parametrize("at", [0, 20_000, -1])
+def test_dense_tail_of_small_probabilities(device, called, dtype, d, at):
+    """One key 2^25.5 above a tail that alone carries V: the output is the
+    tail's share of the sum, to the output's rounding and fp32 sums."""
+    n, share = 40_000, 2.0**-25.5
+    q, k = (torch.zeros((rows, 1, d), dtype=dtype) for rows in (1, n))
+    v = torch.ones((n, 1, d), dtype=dtype)
+    # exact in 16 bits: q.k is 64 x the dominant key's value
+    q[..., 0] = 64.0
+    k[at, :, 0] = -np.log(share) * d**0.5 / 64.0
+    v[at] = 0.0
+    logit = 64.0 * float(k[at, 0, 0]) / d**0.5
+    expected = (n - 1) / (n - 1 + np.exp(logit))
+    out = cope_attention(q.to(device), k.to(device), v.to(device), cope_of(device, torch.zeros((d, 64))),
+                         torch.tensor([n - 1], device=device)).cpu().double().numpy()
+    assert "cs_ccpe_attention" not in called
+    np.testing.assert_allclose(out, expected, rtol=REL[dtype] + n * 2.0**-24 / 32)
