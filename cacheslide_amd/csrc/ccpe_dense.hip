@@ -13,29 +13,40 @@
 // What bounds it.  f32: the matrix cores (v_mfma_f32_32x32x2_f32, 64 of 64
 // cycles for each of the two products of a 32 x 32 tile at D = 128).  16-bit
 // types: the position and softmax arithmetic of the VALU beside the MFMAs of 32
-// cycles (f16 at D = 128: 8 of Q.K and 40 of P.V a tile).  Both are contractions, so a wave that computes one (row,
-// head) pair on scalar dot products -- the generic kernel -- is two orders of
-// magnitude away: at 1000 tokens, 32 query heads over 8 KV heads, D = 128,
-// f16, that kernel took 4150 us and this one takes 88; f32 at 2048 tokens, 16
-// heads over 4, D = 128: a whole call 8.6 ms before, 0.8 ms now.
+// cycles (f16 at D = 128: 8 of Q.K and 40 of P.V a tile), and the latency of a
+// tile's loads: the compiler keeps `kr`, and of f32 also `vr`, in scratch memory
+// (48 bytes a lane for f16 at D = 128, 80 and 144 for f32, none for 16-bit types
+// at D = 64), so that those loads are waited for as they are issued.  Both
+// products are contractions, so a wave that computes one (row, head) pair on
+// scalar dot products -- the generic kernel -- is two orders of magnitude away:
+// at 1000 tokens, 32 query heads over 8 KV heads, D = 128, f16, that kernel
+// took 4150 us and this one takes 86; f32 at 2048 tokens, 16 heads over 4, D =
+// 128: a whole call 8.6 ms before, 0.54 ms now.
 //
 // Decomposition, as in ccpe_prefill.hip: a wave owns 32 (row, head) columns
 // of one GQA group and walks key tiles of 32 from the right-most causal key
 // leftwards; S^T = K Q^T leaves a column's 32 scores on two lanes (n and
 // n + 32), where the suffix sum of the gates and the online softmax are
 // per-lane scalars.  K and V tiles are staged through LDS by the whole
-// workgroup: the next tile's global loads are in registers while this tile is
-// computed, two workgroups per CU cover each other's barriers.  Rows are
-// padded so that the 16-byte K reads of 16 lanes fall in distinct banks.
+// workgroup, the next tile's global loads issued before this tile is computed.
+// Rows are padded so that the 16-byte K reads of 16 lanes fall in distinct
+// banks.  A workgroup has 4 waves at every size, also where a short call leaves
+// compute units idle and where the tables (66 KB at P = 128) leave room for one
+// workgroup per CU: with 2 waves twice as many workgroups share
+// the rows, but each stages its tiles with half the threads, and nothing was
+// gained at any size (17 to 4096 tokens, 40 to 300 rows over 3000 keys).  us a
+// call with 2 and 4 waves: f16, D = 128, 1000 tokens 142 and 135, 4096 636 and
+// 526, P = 128 847 and 690; f32, D = 128, P = 128, 2048 tokens 939 and 692;
+// bf16, D = 64, 40 rows over 3000 keys 186 and 153; 17 f16 tokens 72 and 72.
 //
 // Precision.  Products of the inputs are summed in fp32 and gates in fp64, as
 // in the generic kernel, and a probability keeps its fp32 value whatever its
 // size: f32 multiplies it in fp32, the 16-bit types as three bf16 terms (24
 // bits, the range of fp32) by V in bf16, an f16 V as two bf16 terms, which hold
 // it exactly.  (As two f16 terms a probability ends at 2^-25: 40000 keys below
-// it, 8e-4 of the softmax, left the output but not its norm.  The bf16 terms
-// take 142 us a call at 1000 tokens, 32 heads over 8, D = 128, those 137.)
-// f32 forms gates and exponentials as the generic kernel does; the 16-bit
+// it, 8e-4 of the softmax, left the output but not its norm.  At 1000
+// tokens, 32 heads over 8, D = 128, 2 waves a workgroup, a call took 137 us with
+// those, 142 with the bf16 terms.)  f32 forms gates and exponentials as the generic kernel does; the 16-bit
 // types take v_exp_f32 and v_rcp_f32, within a unit in the last place each, of
 // a score scaled once, where the generic kernel rounds the logit.  The table QE
 // uses fp32 products (f32) or Q and E split into bf16 terms that keep 24 bits
@@ -61,6 +72,8 @@ typedef __attribute__((__vector_size__(4 * sizeof(__bf16)))) __bf16 bf16x4_tr;
 #define CS_LDS __attribute__((address_space(3)))
 
 constexpr int kCols = 32;   // (row, head) columns per wave
+constexpr int kWaves = 4;   // per workgroup: 128 columns share a staged tile
+constexpr int kThreads = 64 * kWaves;
 constexpr int kTileN = 32;  // keys per tile
 constexpr int kMaxPos = 128;
 constexpr float kLog2e = 1.4426950408889634f;
@@ -130,12 +143,11 @@ __device__ inline void split_bf16(float x, __bf16 (&t)[N]) {
 // 8h + 0..7; f32 step 4c + i takes dim 8c + 4h + i, so that a lane reads its
 // half of a K row in 16-byte pieces; P.V takes the scores as they lie, key
 // 8 (v / 4) + 4h + v % 4 for register v.
-template <typename T, int D, int WAVES>
-__global__ void __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(2, 2)))
+template <typename T, int D>
+__global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2)))
 ccpe_dense_kernel(dense_params p) {
   using E = dense_elem<T>;
   constexpr bool kF32 = E::kSize == 4;
-  constexpr int kThreads = 64 * WAVES;
   constexpr int kRow = D * E::kSize + E::kPad;      // bytes of a staged row
   constexpr int kChunks = D * E::kSize / 16;        // 16-byte chunks of a row
   constexpr int kLoads = kTileN * kChunks / kThreads;
@@ -504,36 +516,16 @@ ccpe_dense_kernel(dense_params p) {
   if (__any(huge && row_ok) && lane == 0) atomicOr(p.flags, CS_FLAG_POLICY_GENERIC);
 }
 
-int compute_units() {
-  static int cus[64] = {};
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
-  if (cus[dev] == 0) {
-    int v = 0;
-    cus[dev] = hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && v > 0 ? v : 256;
-  }
-  return cus[dev];
-}
-
 template <typename T, int D>
 int launch_dense(dense_params p, hipStream_t s) {
-  // 4 waves per workgroup (128 columns share a staged tile) once that gives
-  // three workgroups per two CUs, else 2 waves: a short call's longest walks
-  // are then spread over twice as many workgroups.
-  const auto blocks = [&](int w) { return ceil_div(p.nq, kCols * w / p.group) * p.hkv; };
-  const int waves = blocks(4) < 3 * compute_units() / 2 ? 2 : 4;
-  p.rows_per_wg = kCols * waves / p.group;
-  const int64_t total = blocks(waves);
+  p.rows_per_wg = kCols * kWaves / p.group;
+  const int64_t total = ceil_div(p.nq, p.rows_per_wg) * p.hkv;
   CS_REQUIRE(total < (1ll << 31), "grid too large");
   p.row_blocks = static_cast<int32_t>(total / p.hkv);
   p.tab_stride = (p.npos + 1) | 1;  // entries 0 .. P, an odd number of words
   const size_t smem = (1 + dense_elem<T>::kVTiles) * kTileN * (D * dense_elem<T>::kSize + dense_elem<T>::kPad) +
-                      sizeof(float) * kCols * waves * static_cast<size_t>(p.tab_stride);
-  const dim3 grid(static_cast<uint32_t>(total)), block(64 * waves);
-  if (waves == 2)
-    hipLaunchKernelGGL((ccpe_dense_kernel<T, D, 2>), grid, block, smem, s, p);
-  else
-    hipLaunchKernelGGL((ccpe_dense_kernel<T, D, 4>), grid, block, smem, s, p);
+                      sizeof(float) * kCols * kWaves * static_cast<size_t>(p.tab_stride);
+  hipLaunchKernelGGL((ccpe_dense_kernel<T, D>), dim3(static_cast<uint32_t>(total)), dim3(kThreads), smem, s, p);
   CS_LAUNCH_CHECK("ccpe_dense");
   return CS_OK;
 }

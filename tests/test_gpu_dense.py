@@ -69,17 +69,26 @@ def test_dense_tables_strides_and_sparse_rows(device, called, dtype, npos):
     assert "cs_ccpe_attention" not in called
 
 
-def test_dense_wide_workgroups(device, called):
-    """Enough row blocks for the 4-wave workgroups."""
-    check(device, torch.float16, 64, 32, 32, 2100, np.arange(2000, 2100), 64, seed=5)   # 2 waves
+def test_dense_many_workgroups(device, called):
+    """More row blocks than compute units, the same rows alone in a few."""
+    check(device, torch.float16, 64, 32, 32, 2100, np.arange(2000, 2100), 64, seed=5)
     rng = torch.Generator().manual_seed(9)
     q, k, v = (torch.randn((2100, 32, 64), generator=rng).half().to(device) for _ in range(3))
     cope = cope_of(device, seeded((64, 64), 4, scale=0.1))
     rows = torch.arange(2100, device=device)
-    wide = cope_attention(q, k, v, cope, rows)                  # 525 four-wave blocks
+    wide = cope_attention(q, k, v, cope, rows)                  # 544 workgroups
     few = torch.arange(1000, 1130, device=device)
     torch.testing.assert_close(wide[few], cope_attention(q[few], k, v, cope, few), rtol=0, atol=2.0**-9)
     assert "cs_ccpe_attention" not in called
+
+
+@pytest.mark.parametrize("dtype,d", [(torch.float16, 128), (torch.float16, 64), (torch.float32, 128),
+                                     (torch.float32, 64), (torch.bfloat16, 64)])
+@pytest.mark.parametrize("hq,hkv", [(4, 1), (2, 2)])
+def test_dense_largest_table(device, called, dtype, d, hq, hkv):
+    """128 positions (one workgroup per CU) and rows past a workgroup's last."""
+    check(device, dtype, d, hq, hkv, 421, np.arange(421), 128, seed=hq)
+    assert "cs_ccpe_attention_dense" in called and "cs_ccpe_attention" not in called
 
 
 def test_dense_values_past_the_range_take_the_generic_kernel(device, called):
