@@ -1097,11 +1097,15 @@ extern "C" int64_t cs_ccpe_decode_workspace_bytes(int32_t batch, int32_t hq, int
 extern "C" int64_t cs_ccpe_decode_workspace_best_bytes(int32_t batch, int32_t hq, int32_t max_nk,
                                                        int32_t split) {
   if (batch <= 0 || hq <= 0 || max_nk <= 0 || split <= 0) return 0;
-  // the finest plan of any call of this size: fewest KV heads, smallest split 0
-  const split_plan f = plan_splits(batch, hq, hq < kMaxGroup ? 1 : hq / kMaxGroup, max_nk, split, 2, -1);
-  const int64_t fine = static_cast<int64_t>(batch) * hq * f.smax * kSplitBytes;
-  const int64_t base = cs_ccpe_decode_workspace_bytes(batch, hq, max_nk, split);
-  return fine > base ? fine : base;
+  // the finest plan of any call of this size: fewest KV heads, and every split 0
+  // that a position count gives (4 P in steps of 64: a larger one can leave room
+  // for another halving within the most splits)
+  int64_t smax = ceil_div(max_nk, split);
+  for (int32_t npos = 64; npos <= kMaxPos; npos += 16) {
+    const split_plan f = plan_splits(batch, hq, hq < kMaxGroup ? 1 : hq / kMaxGroup, max_nk, split, npos, -1);
+    smax = f.smax > smax ? f.smax : smax;
+  }
+  return static_cast<int64_t>(batch) * hq * smax * kSplitBytes;
 }
 
 namespace {
