@@ -15,9 +15,13 @@ from cacheslide_amd.decode_model import DecoderShape, PagedDecoder
 pytestmark = pytest.mark.gpu
 
 
-def run(device, shape, b, bs, fused, monkeypatch, positions=None, cols=6):
+def run(device, shape, b, bs, fused, monkeypatch, positions=None, cols=6, max_context=None):
     monkeypatch.setattr(dm, "FUSED_BATCH", 32 if fused else 0)
     model = PagedDecoder(shape, device, seed=3, std=0.05)
+    # the weights of every norm, as built all ones, distinct
+    scales = torch.Generator(device=device).manual_seed(5)
+    for norm in [model.norm, *(w for layer in model.layers for w in (layer.in_norm, layer.post_norm))]:
+        norm.normal_(1.0, 0.5, generator=scales)
     gen = torch.Generator(device=device).manual_seed(4)
     wide = [torch.empty((b * cols + 1, shape.kv_heads, bs, 256), dtype=torch.bfloat16, device=device).normal_(
         generator=gen) for _ in range(shape.layers)]
@@ -26,9 +30,17 @@ def run(device, shape, b, bs, fused, monkeypatch, positions=None, cols=6):
     ids = (torch.arange(b, device=device) * 7) % shape.vocab
     if positions is None:
         positions = (torch.arange(b, device=device) * 13) % (cols * bs)
+    before = [cache.clone() for cache in wide]
     flags = _hip.new_flags(device)
-    logits = model.step(ids, positions, wide, table, max_context=cols * bs, flags=flags,
-                        workspace=decode_workspace(b, shape.heads, cols * bs, 1024, device))
+    max_context = cols * bs if max_context is None else max_context
+    logits = model.step(ids, positions, wide, table, max_context=max_context, flags=flags,
+                        workspace=decode_workspace(b, shape.heads, max_context, 1024, device))
+    # only the records of new tokens inside the table may differ
+    for cache, old in zip(wide, before):
+        for i, pos in enumerate(positions.tolist()):
+            if pos < cols * bs:
+                old[table[i, pos // bs], :, pos % bs] = cache[table[i, pos // bs], :, pos % bs]
+        assert torch.equal(cache, old)
     return logits, wide, flags
 
 
@@ -49,7 +61,6 @@ def test_fused_step_matches_library_step(device, monkeypatch, b, heads, kv, ffn,
         return (x.double() - y.double()).norm() <= 2e-2 * y.double().norm()
     assert got.shape == want.shape and close(got, want)
     for x, y in zip(got_cache, want_cache):
-        # records other than the new tokens' are untouched
         same = (x == y).all(-1)
         assert int((~same).sum()) <= b * kv and close(x, y)
 
@@ -57,7 +68,9 @@ def test_fused_step_matches_library_step(device, monkeypatch, b, heads, kv, ffn,
 def test_a_position_past_the_table_is_flagged_and_skipped(device, monkeypatch):
     shape = DecoderShape(layers=1, hidden=256, heads=2, kv_heads=1, ffn=64, vocab=64, npos=16)
     positions = torch.tensor([3, 96], device=device)       # six blocks of 16: keys 0..95
-    got, cache, flags = run(device, shape, 2, 16, True, monkeypatch, positions=positions)
-    assert torch.isfinite(cache[0].float()).all()
+    # a context of 97 keys is allowed, so that only the missing block is reported
+    _, _, flags = run(device, shape, 2, 16, True, monkeypatch, positions=positions, max_context=112)
+    assert _hip.read_flags(flags)[0] & _hip.FLAG_BLOCK_INVALID
+    assert not _hip.read_flags(flags)[0] & _hip.FLAG_CONTEXT_RANGE
     with pytest.raises(ValueError):
         raise_flags(flags)
