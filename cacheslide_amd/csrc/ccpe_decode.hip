@@ -98,18 +98,6 @@ struct decode_params {
   const int32_t* gate;
 };
 
-// Compute units of the current device (cached per device; 256 without one).
-int compute_units() {
-  static int cus[64] = {};
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
-  if (cus[dev] == 0) {
-    int v = 0;
-    cus[dev] = hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && v > 0 ? v : 256;
-  }
-  return cus[dev];
-}
-
 __device__ inline int64_t ws_index(const decode_params& p, int b, int h, int r) {
   return (static_cast<int64_t>(b) * p.hq + h) * p.smax + r;
 }

@@ -962,18 +962,6 @@ int side_lane_of_current(side_lane** out) {
   return CS_OK;
 }
 
-// Compute units of the current device (cached per device).
-int device_cus() {
-  static int cus[64] = {};
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
-  if (cus[dev] == 0) {
-    int v = 0;
-    cus[dev] = hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && v > 0 ? v : 256;
-  }
-  return cus[dev];
-}
-
 int fill_kv(const cs_kv_source* kv, cs::kv_addr* a) {
   CS_REQUIRE(kv != nullptr, "null kv source");
   cs::kv_addr r{};
@@ -1100,7 +1088,7 @@ int prepare_prefill(const void* q, int64_t q_s_batch, int64_t q_s_tok, int64_t q
   // than the balance gives: 5 requests of 333 rows (440 workgroups) 198 us
   // against 138, 2000 rows of one (504) 129 against 109; 1000 rows (256) 74
   // against 78.
-  if (static_cast<int64_t>(batch) * hkv * ceil_div(nq, kCols * 4 / group) < 3 * device_cus() / 2 &&
+  if (static_cast<int64_t>(batch) * hkv * ceil_div(nq, kCols * 4 / group) < 3 * compute_units() / 2 &&
       2 * (tab_bytes(2) + kStaticLds) <= kLdsLimit)
     waves = 2;
   // a caller with few rows per workgroup (one per request) asks for narrow ones

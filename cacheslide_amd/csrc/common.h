@@ -15,6 +15,9 @@ namespace cs {
 // ---------------------------------------------------------------- errors
 void set_error(const char* fmt, ...);
 
+// Compute units of the current device (cached per device; 256 without one).
+int compute_units();
+
 #define CS_REQUIRE(cond, ...)            \
   do {                                   \
     if (!(cond)) {                       \
