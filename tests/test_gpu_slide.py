@@ -128,6 +128,23 @@ def test_free_list_bits_left_after_acquire(device, nbits, count):
     np.testing.assert_array_equal(fl.free_mask().numpy(), left)
 
 
+@pytest.mark.parametrize("nbits", [131_072, 131_073, 300_007])
+@pytest.mark.parametrize("share", [0.01, 0.3, 0.5, 1.0])
+def test_free_list_of_any_density(device, nbits, share):
+    """Words that each lane writes and words that their wave writes, within and
+    past a round of 4096 words, with a last word taken in part."""
+    rng = np.random.default_rng(nbits)
+    free = rng.random(nbits) < share
+    free[40_000:44_000] = rng.random(4_000) < 0.9        # both kinds in one round
+    fl = relocate.SlotFreeList(nbits, device, free_from=nbits)
+    fl.release(torch.from_numpy(np.flatnonzero(free)).to(device))
+    for count in (1, int(free.sum()) // 3, int(free.sum()) // 2):
+        want = np.flatnonzero(free)[:count]
+        np.testing.assert_array_equal(fl.acquire(count).cpu().numpy(), want)
+        free[want] = False
+        np.testing.assert_array_equal(fl.free_mask().numpy(), free)
+
+
 @pytest.mark.parametrize("shape", [(2, 9, 3, 4, 8), (3, 9, 8, 16, 256), (7, 2, 16, 96), (9, 1, 16, 128), (9, 1, 17, 120)])
 def test_page_copy_of_compact_pages(device, shape):
     """Pages that are one run of bytes, of less than, exactly and more than the
