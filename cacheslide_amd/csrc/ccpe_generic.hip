@@ -589,10 +589,11 @@ __global__ void __launch_bounds__(256) policy_lower_kernel(cs_policy_lower_args 
   if (__syncthreads_or(descents)) {
     __shared__ int64_t part[256];
     for (int64_t base = 0; base < a.n_selected; base += 256) {
-      const int n = static_cast<int>(a.n_selected - base < 256 ? a.n_selected - base : 256);
-      if (static_cast<int>(threadIdx.x) < n) part[threadIdx.x] = a.selected[base + threadIdx.x];
+      const int64_t t = base + threadIdx.x;
+      part[threadIdx.x] = t < a.n_selected ? a.selected[t] : a.selected[base];
       __syncthreads();
-      for (int t = 0; t < n; ++t) found = found || part[t] == q;
+#pragma unroll 32
+      for (int u = 0; u < 256; ++u) found |= part[u] == q;
       __syncthreads();
     }
   } else {
