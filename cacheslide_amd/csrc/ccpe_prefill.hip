@@ -1075,19 +1075,21 @@ int prepare_prefill(const void* q, int64_t q_s_batch, int64_t q_s_tok, int64_t q
   p.group = group;
   // fp32 QE table rows of an odd number of words (no bank conflicts between
   // columns).  4 wavefronts (128 columns) while two such workgroups fit in a
-  // CU, so one workgroup's prologue and barriers overlap the other's tile
-  // loop; else 8 wavefronts (one workgroup, still two waves per SIMD) while
-  // its table fits, else 4.
+  // CU (P <= 54), so one workgroup's prologue and barriers overlap the other's
+  // tile loop; else 8 wavefronts (one workgroup, still two waves per SIMD) while
+  // its table fits (P <= 106), else 4.
   // P + 1 entries per column (entry P repeats P-1), an odd number of words
   const int tab_stride = (max_positions + 1) | 1;
   auto tab_bytes = [&](int w) { return sizeof(float) * kCols * w * static_cast<size_t>(tab_stride); };
   int waves = 2 * (tab_bytes(4) + kStaticLds) <= kLdsLimit ? 4 : (tab_bytes(8) + kStaticLds <= kLdsLimit ? 8 : 4);
   // A launch of fewer 4-wave workgroups than three per two CUs (a selective
   // call's few hundred rows) runs 2-wave workgroups: twice as many workgroups
-  // share the longest key walks.  With more, the half-used tiles cost more
-  // than the balance gives: 5 requests of 333 rows (440 workgroups) 198 us
-  // against 138, 2000 rows of one (504) 129 against 109; 1000 rows (256) 74
-  // against 78.
+  // share the longest key walks.  With more, the half-used tiles cost more than
+  // the balance gives.  us a call with 2 / 4 / 8 wavefronts, the counts in 4-wave
+  // workgroups, P = 64: 5 requests of 333 rows (440) 189 / 174 / 129, 2000 rows
+  // of one (504) 124 / 110 / 105, 1000 rows (256) 73 / 71 / 78, 100 rows of four
+  // (128) 145 / 140 / 155; P = 16, the 440: 183 / 117 / 126.  Where two 2-wave
+  // workgroups do not fit a CU (P > 110) the launch keeps its 4.
   if (static_cast<int64_t>(batch) * hkv * ceil_div(nq, kCols * 4 / group) < 3 * compute_units() / 2 &&
       2 * (tab_bytes(2) + kStaticLds) <= kLdsLimit)
     waves = 2;
@@ -1643,7 +1645,10 @@ extern "C" int cs_ccpe_prefill_policy_bf16(const cs_ccpe_args* a, void* workspac
   src.v_s_head = vv.stride[1];
   // With selected rows and a profile (an unsplit walk), the call takes the time
   // of its few row blocks that see every key: 4 wavefronts a workgroup leave
-  // each a SIMD of its own (512 tiles: 561 us; 8 wavefronts 620, 2 646).
+  // each a SIMD of its own.  us a call with 2 / 4 / 8, fixed and recomputed keys,
+  // 32 heads over 8, P = 64: 16128 + 256 803 / 707 / 784, 8000 + 256 472 / 424 /
+  // 479, 4000 + 64 337 / 308 / 304, 2000 + 250 238 / 226 / 243, 400 + 64 170 / 172
+  // / 180 (calls of few rows take 2 by the rule for small launches).
   const int max_waves = canon && a->sel_rows ? 4 : 8;
   cs::prefill_params p{};
   int waves = 4;
@@ -1682,9 +1687,10 @@ extern "C" int cs_ccpe_prefill_policy_bf16(const cs_ccpe_args* a, void* workspac
   }
   // Key splits of the row blocks that walk every causal key (planned on the
   // device from the rows' positions and the selected set), when no checker
-  // runs beside the attention: with one, the two kernels already fill the
-  // device, the checker's reads bound the call, and the split parts only take
-  // compute units from it (1.39 against 1.30 ms per reuse call at 16k keys).
+  // runs beside the attention.  With one they were measured when the checker's
+  // reads bound the call and the parts only took compute units from it (1.39
+  // against 1.30 ms per reuse call at 16k keys); the checker has since fallen
+  // from 784 to 180 us, and the line has not been moved.
   const bool split = w.split && !canon && !no_split();
   if (split) {
     p.split_extra = kSplitExtra;
