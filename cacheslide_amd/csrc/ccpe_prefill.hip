@@ -164,7 +164,9 @@ __device__ __forceinline__ void prefill_workgroup(const prefill_params& p, const
     }
   };
   load_e(0);
-  const int64_t qp = row_ok ? qp_raw : -1;
+  // 32 bits below hold any position: one past INT32_MAX - 1 is past every key
+  constexpr int64_t kFarthest = INT32_MAX - 1;
+  const int64_t qp = row_ok ? (qp_raw < kFarthest ? qp_raw : kFarthest) : -1;
   bool sel_col = false;   // the column's row is selected: fixed keys other than its own are invisible
   float canon_self = 0.f;  // canonical position of the column's own key (NaN: contextual)
   // a fixed row that is not selected: its profile row, canonical positions

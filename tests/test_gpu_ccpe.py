@@ -513,6 +513,18 @@ def test_prefill_large_table_and_sparse_rows(device, npos):
     assert_close_bf16(actual, expected)
 
 
+def test_prefill_rows_past_every_key(device):
+    """Query positions past the keys, up to the largest int64, see all of them."""
+    hq, hkv, n, npos = 8, 2, 90, 64
+    q, k, v = (seeded((n, heads, 128), 40 + i, dtype=torch.bfloat16) for i, heads in enumerate((hq, hkv, hkv)))
+    e = seeded((128, npos), 43, scale=0.1)
+    rows = np.arange(n)
+    rows[[5, 40, 77]] = 2**63 - 1, 2**31 + 7, 5000
+    out = cope_attention(q.to(device), k.to(device), v.to(device), cope_on(device, 128, npos, table=e),
+                         torch.from_numpy(rows).to(device))
+    assert_close_bf16(out, orc.cope_attention(acc_np(q), acc_np(k), acc_np(v), e.numpy(), rows))
+
+
 def test_mfma_prefill_zero_table_is_sdpa(device):
     """Library reduction: E = 0 gives causal softmax attention (torch SDPA, fp32, CPU)."""
     n, hq, hkv = 333, 8, 2
