@@ -999,6 +999,9 @@ __global__ void __launch_bounds__(kThreads) decode_finish_kernel(decode_params p
   bool bad = false;
   if (own > 0) {
     if (own >= splits) return;
+    const int lane = threadIdx.x & 63;
+    if (!__any(lane < G && p.tot[ws_index(p, b, h0 + (lane < G ? lane : 0), 0)] < static_cast<double>(p.npos - 1)))
+      return;  // split 0 reaches P-1 for every head: nothing is recomputed
     plan_group<G>(p, s, b, h0, splits, own);
     __syncthreads();
     if (own >= __builtin_amdgcn_readfirstlane(s.fix_end)) return;
