@@ -1555,6 +1555,8 @@ int launch_states(const cs::prefill_params& p, int waves, size_t smem, hipStream
 // Two calls that write softmax states; either may have no rows.  One launch
 // when both run 2-wave workgroups and do not fill the chip (at 32 requests over
 // eight 1024-token runs: 25 and 20 us one after the other, 30 us together).
+// Past 110 positions the runs take 4 waves (prepare_prefill), so they and the
+// tails are two launches.
 int launch_prefill_states_pair(const prefill_states_call& first, const prefill_states_call& second, hipStream_t s) {
   cs::prefill_params p[2];
   int waves[2] = {0, 0};
