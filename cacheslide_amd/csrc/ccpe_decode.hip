@@ -794,7 +794,7 @@ __device__ bool fixup_one(const decode_params& p, smem_t<G>& s, int b, int kvh, 
   make_ctx(p, b, kvh, own, c);
   run_exact<G, PAGED>(p, s, c, false, bad);
   // Every wave's stores have reached this XCD's L2, which one wave then writes
-  // back before the count (a write-back per wave made 128 such workgroups 5 us
+  // back before the count (a write-back per wave made 128 such workgroups 8 us
   // slower); the last workgroup drops what it holds of the others' lines.
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   __syncthreads();
