@@ -121,8 +121,9 @@ def _rows(name: str, tensor: Tensor, ck: _Checks, bit: int) -> None:
 def _positions(
     name: str, tensor: Tensor, n: int, device: torch.device, ck: _Checks, is_key: bool,
     exc: type = ValueError,
-) -> None:
-    """position.py:127-137: nonnegative distinct int64 [n] on the device."""
+) -> Tensor:
+    """position.py:127-137: nonnegative distinct int64 [n] on the device;
+    returned contiguous, as the kernels read them."""
     if (
         not isinstance(tensor, Tensor)
         or tensor.ndim != 1
@@ -131,11 +132,13 @@ def _positions(
         or tensor.device != device
     ):
         ck.fail(exc(f"{name} must be nonnegative int64 [{n}] on {device}"))
+    tensor = tensor.contiguous()
     ck.lists[1 if is_key else 0] = tensor
     neg = _hip.FLAG_KPOS_NEGATIVE if is_key else _hip.FLAG_QPOS_NEGATIVE
     dup = _hip.FLAG_KPOS_DUPLICATE if is_key else _hip.FLAG_QPOS_DUPLICATE
     ck.device_step(neg, exc, f"{name} must be nonnegative int64 [{n}] on {device}")
     ck.device_step(dup, exc, f"{name} must identify distinct token positions")
+    return tensor
 
 
 def _qk_layout(query: Tensor, key: Tensor, ck: _Checks) -> None:
@@ -198,13 +201,14 @@ def validate_contextual_path(
     ck.device_step(_hip.FLAG_POS_NONFINITE, CCPEPositionError, message)
     if isinstance(atol, bool) or not isinstance(atol, (int, float)) or not math.isfinite(atol) or atol < 0:
         ck.fail(CCPEPositionError("atol must be finite and nonnegative"))
+    lists = []
     for name, coordinates, size, is_key in (
         ("query_positions", query_positions, positions.shape[1], False),
         ("key_positions", key_positions, positions.shape[2], True),
     ):
         if not isinstance(coordinates, Tensor):
             ck.fail(CCPEPositionError(f"{name} must be an int64 tensor"))
-        _positions(name, coordinates, size, device, ck, is_key, exc=CCPEPositionError)
+        lists.append(_positions(name, coordinates, size, device, ck, is_key, exc=CCPEPositionError))
     ck.device_step(_hip.FLAG_KPOS_UNSORTED, CCPEPositionError, "key_positions must be strictly increasing")
     if attention_mask is not None:
         if (
@@ -217,7 +221,7 @@ def validate_contextual_path(
             ck.fail(CCPEPositionError("attention_mask must be bool [query,key] or [head,query,key]"))
     mask = _mask_view(attention_mask, positions.shape[1], positions.shape[2])
     call(
-        "cs_validate_contextual_path", vref(positions), ptr(query_positions), ptr(key_positions),
+        "cs_validate_contextual_path", vref(positions), ptr(lists[0]), ptr(lists[1]),
         vref(mask), float(atol), ck.flags_ptr, ck.stream,
     )
     for bit, text in _PATH_MESSAGES:
@@ -411,10 +415,10 @@ class CoPE(nn.Module):
         device = _device_of(query)
         ck = _Checks(device)
         _qk_layout(query, key, ck)
-        _positions("query_positions", query_positions, query.shape[0], device, ck, False)
+        query_positions = _positions("query_positions", query_positions, query.shape[0], device, ck, False)
         if key_positions is None:
             key_positions = torch.arange(key.shape[0], device=device)
-        _positions("key_positions", key_positions, key.shape[0], device, ck, True)
+        key_positions = _positions("key_positions", key_positions, key.shape[0], device, ck, True)
         ck.device_step(_hip.FLAG_KPOS_UNSORTED, ValueError,
                        "key_positions must be strictly increasing for reverse cumsum")
         mask = _checked_mask(attention_mask, query, key, ck)
@@ -559,10 +563,10 @@ def cope_attention(
         if visibility_mask is not None:
             ck.fail(ValueError("visibility_transform and visibility_mask are mutually exclusive"))
     nq, hq, nk = query.shape[0], query.shape[1], key.shape[0]
-    _positions("query_positions", query_positions, nq, device, ck, False)
+    query_positions = _positions("query_positions", query_positions, nq, device, ck, False)
     default_keys = key_positions is None   # coordinates 0..nk-1: nothing to check
     if not default_keys:
-        _positions("key_positions", key_positions, nk, device, ck, True)
+        key_positions = _positions("key_positions", key_positions, nk, device, ck, True)
     for name, mask in (("attention_mask", attention_mask), ("visibility_mask", visibility_mask)):
         if mask is not None and mask.shape not in ((nq, nk), (1, nq, nk), (hq, nq, nk)):
             ck.fail(ValueError(f"{name} has an incompatible full-query shape"))

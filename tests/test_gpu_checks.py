@@ -61,3 +61,21 @@ def test_selected_rows_and_fixed_keys(device, m, ordered):
                                      rows.to(device), None if keys is None else keys.to(device), 1000)
         assert torch.equal(sel.cpu().bool(), torch.isin(rows, selected))
         assert torch.equal(fix.cpu().bool(), torch.isin(want_keys, torch.tensor(fixed)))
+
+
+@pytest.mark.parametrize("dtype,d", [(torch.bfloat16, 128), (torch.float16, 64), (torch.float64, 64)])
+@pytest.mark.parametrize("with_keys", [False, True])
+def test_strided_position_lists(device, dtype, d, with_keys):
+    n = 60
+    cope = CoPE(d, 16, device=device)
+    with torch.no_grad():
+        cope.position_embeddings.copy_(seeded((d, 16), 5, scale=0.1))
+    q, k, v = (seeded((n, 2, d), i, dtype=dtype).to(device) for i in range(3))
+    rows = torch.arange(n, device=device).flip(0).contiguous()
+    keys = 2 * torch.arange(n, device=device) if with_keys else None
+    spread = lambda x: None if x is None else torch.stack([x, x + 7], 1)[:, 0]  # noqa: E731
+    assert spread(rows).stride(0) == 2
+    want = cope_attention(q, k, v, cope, rows, keys)
+    assert torch.equal(cope_attention(q, k, v, cope, spread(rows), spread(keys)), want)
+    logits = cope(q, k, rows, keys)
+    assert torch.equal(cope(q, k, spread(rows), spread(keys)), logits)
