@@ -77,3 +77,31 @@ def test_splits_recomputed_side_by_side(device, lens, hq, hkv, npos, low_gates):
     for _ in range(20):
         workspace.fill_(0xFF)
         assert torch.equal(ccpe_decode_paged(*args, max_context=max(lens), workspace=workspace), first)
+
+
+def test_recomputed_splits_under_graph_replay(device):
+    """The count of recomputed splits is cleared by every replay of a call,
+    also between eager calls of the same workspace."""
+    lens = [1500, 300]
+    args, want = setup(device, lens, 8, 2, 64, low_gates=0.35)
+    workspace = decode_workspace(2, 8, 1500, 1024, device)
+    flags, out = _hip.new_flags(device), torch.empty((2, 8, 128), dtype=torch.bfloat16, device=device)
+    run = lambda: ccpe_decode_paged(*args, max_context=1500, workspace=workspace, flags=flags, out=out,  # noqa: E731
+                                    check=False)
+    run()
+    torch.cuda.synchronize()
+    eager = out.clone()
+    assert_close_bf16(eager, want)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        run()
+    for _ in range(4):
+        out.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, eager)
+        out.zero_()
+        run()
+        torch.cuda.synchronize()
+        assert torch.equal(out, eager)
+    assert _hip.read_flags(flags)[0] == 0
