@@ -20,7 +20,7 @@
 // products are contractions, so a wave that computes one (row, head) pair on
 // scalar dot products -- the generic kernel -- is two orders of magnitude away:
 // at 1000 tokens, 32 query heads over 8 KV heads, D = 128, f16, that kernel
-// took 4150 us and this one takes 86; f32 at 2048 tokens, 16 heads over 4, D =
+// took 4150 us and this one takes 81; f32 at 2048 tokens, 16 heads over 4, D =
 // 128: a whole call 8.6 ms before, 0.54 ms now.
 //
 // Decomposition, as in ccpe_prefill.hip: a wave owns 32 (row, head) columns
@@ -46,7 +46,9 @@
 // it exactly.  (As two f16 terms a probability ends at 2^-25: 40000 keys below
 // it, 8e-4 of the softmax, left the output but not its norm.  At 1000
 // tokens, 32 heads over 8, D = 128, 2 waves a workgroup, a call took 137 us with
-// those, 142 with the bf16 terms.)  f32 forms gates and exponentials as the generic kernel does; the 16-bit
+// those, 142 with the bf16 terms; with 4 waves, and each term of P multiplied by
+// all of V before the next so that consecutive products are independent, 131.)
+// f32 forms gates and exponentials as the generic kernel does; the 16-bit
 // types take v_exp_f32 and v_rcp_f32, within a unit in the last place each, of
 // a score scaled once, where the generic kernel rounds the logit.  The table QE
 // uses fp32 products (f32) or Q and E split into bf16 terms that keep 24 bits
@@ -463,17 +465,22 @@ ccpe_dense_kernel(dense_params p) {
           for (int w = 0; w < 3; ++w) pb[w][i] = t[w];
         }
 #pragma unroll
-        for (int db = 0; db < kDb; ++db)
+        for (int u = E::kVTiles - 1; u >= 0; --u) {
+          bf16x8 va[kDb];
 #pragma unroll
-          for (int u = E::kVTiles - 1; u >= 0; --u) {
+          for (int db = 0; db < kDb; ++db) {
             const char* at = vrd16 + u * kTileN * kRow + 16 * ks * kRow + 64 * db;
             const bf16x4_tr lo = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((CS_LDS bf16x4_tr*)at);
             const bf16x4_tr hi = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((CS_LDS bf16x4_tr*)(at + 8 * kRow));
-            const auto va = __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
-            // third term of P times second of V: below 2^-26 of the product
-#pragma unroll
-            for (int w = 2 - u; w >= 0; --w) o[db] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(va, pb[w], o[db], 0, 0, 0);
+            va[db] = __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
           }
+          // third term of P times second of V: below 2^-26 of the product
+#pragma unroll
+          for (int w = 2 - u; w >= 0; --w)
+#pragma unroll
+            for (int db = 0; db < kDb; ++db)
+              o[db] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(va[db], pb[w], o[db], 0, 0, 0);
+        }
       }
     }
   };
