@@ -378,12 +378,12 @@ __global__ void __launch_bounds__(kAcqThreads)
     return;
   }
   if (tid == 0) *status = CS_OK;
-  int64_t room = count;  // slots still to be taken before this round
+  int64_t room = count;  // slots still to be taken
   for (int64_t base = 0; base < words && room > 0; base += kRound) {
     uint32_t bits[kAcqWords];
 #pragma unroll
     for (int k = 0; k < kAcqWords; ++k) bits[k] = next[k];
-    load(base + kRound, next);  // in flight during this round
+    load(base + kRound, next);  // in flight while these are ranked
     int rank[kAcqWords];
 #pragma unroll
     for (int k = 0; k < kAcqWords; ++k) {
@@ -409,7 +409,7 @@ __global__ void __launch_bounds__(kAcqThreads)
     for (int k = 0; k < kAcqWords; ++k) rank[k] += __shfl(upto - sum, kAcqWaves * k + wave, 64);
     const int round = __shfl(upto, 63, 64);
     __syncthreads();  // sums is written again in the next round
-    // ranks are relative to this round's first; those below `room` are taken
+    // ranks count from the first free bit at `base`; those below `room` are taken
     int64_t* slots = out + (count - room);
 #pragma unroll
     for (int k = 0; k < kAcqWords; ++k) {
